@@ -114,10 +114,10 @@ int t81_hip_ternary_matmul_kernel(int which, const void *x, int x_dtype, const u
  * multiple of 16, or bf16 ones with K not a multiple of 8, and workspace_bytes is at least
  * t81_hip_ternary_matmul_workspace_size(...), K is split over several workgroups
  * per tile: each writes its partial tile to the workspace and a second kernel sums
- * the partials in split order (deterministic).  With float32 activations past 64 tokens
- * (K % 8 == 0) the workspace may instead hold the activations' bf16 hi and lo planes,
- * chunk by chunk, and each chunk runs as two bf16 launches (the second adding the lo
- * plane's product to C).  NULL / 0 bytes: no split, no planes.  The workspace must be
+ * the partials in split order (deterministic).  With float32 activations past 32 tokens the
+ * workspace holds the activations' bf16 hi and lo planes (chunk by chunk of the tokens, or
+ * part by part of K, where they are large) and such partials, and one launch per chunk
+ * sums both planes' products.  NULL / 0 bytes: no split, no planes.  The workspace must be
  * 16-byte aligned and not used by another call at the same time.
  * Replaces: the same reference interfaces as t81_hip_ternary_matmul; the
  *           reference's CPU path needs no workspace, so it has no such argument. */

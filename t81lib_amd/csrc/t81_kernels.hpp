@@ -108,6 +108,13 @@ hipError_t launch_gemm(const void *x, int x_dtype, const uint8_t *w, void *c, in
                        hipStream_t s, void *ws = nullptr, int64_t ws_bytes = 0);
 int64_t gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, int x_dtype);
 
+// gemm_planes.hip (K3, float32 activations as bf16 planes in the workspace): the workspace
+// a shape uses (0: it does not take the shape) and the launch, given that much.
+int64_t gemm_planes_workspace_bytes(int64_t m, int64_t n, int64_t k);
+hipError_t launch_gemm_planes(const float *x, const uint8_t *w, float *c, int64_t m, int64_t n,
+                              int64_t k, float alpha, float beta, const float *bias,
+                              hipStream_t s, void *ws);
+
 // gemm_i8.hip (K3, int8 activations, integer matrix cores): whether a shape takes it, the
 // workspace its split-K plan uses, and the launch (C int32; accumulate: C += product)
 bool gemm_i8_fits(const void *x, int64_t m, int64_t n, int64_t k);
