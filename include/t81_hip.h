@@ -328,6 +328,41 @@ int t81_hip_spmm_simple(const int64_t *values, const int32_t *row_idx, const int
                         int64_t nnz, int rows, int cols, const float *B, float *C, int N,
                         float alpha, float beta, void *stream);
 
+/* ---- quantization-aware training (t8.nn.Linear in train mode) ----
+ * The weight passes and products of F.linear(x, ternary(w / s) * s, b) and its backward, with
+ * s in device memory.  w_dtype: T81_DTYPE_F32 / BF16 / F16; every operation rounds to that
+ * type, as the tensor expressions it replaces do. */
+
+/* *scale = max(max |w|, 1e-6) over count > 0 values (rounded to w's type; NaN if any is);
+ * with previous given, max(0.99 * *previous + 0.01 * that, 1e-6).  scratch: 4096 bytes.
+ * Replaces: Linear._update_training_scale, t81/nn/linear.py:72-85. */
+int t81_hip_qat_scale(const void *w, int w_dtype, int64_t count, const float *previous,
+                      float *scale, void *scratch, void *stream);
+
+/* u = w / *scale; q = sign(u) where min(|u|, 1) >= threshold, else 0; wq = q * *scale (w's
+ * type, rows x cols), packed = q in limbs, inner (rows x ceil(cols / 48) x 4 uint16): bit i of
+ * a word says that -0.5 < u < 0.5 (or NaN) at that column 12 q + i of the limb.
+ * Replaces: ternary(w / s) * s, t81/nn/linear.py:93-99, t81/qat.py:12-46. */
+int t81_hip_qat_quantize(const void *w, int w_dtype, const float *scale, float threshold,
+                         void *wq, uint8_t *packed, uint16_t *inner, int64_t rows, int64_t cols,
+                         void *stream);
+
+/* out = inner ? ((g * *scale) * 2) / *scale : 0, the gradient of the above for w; out may be g.
+ * Replaces: the backward of the same expression (dorso_round, t81/qat.py:28-35). */
+int t81_hip_qat_weight_grad(const void *g, int g_dtype, const float *scale,
+                            const uint16_t *inner, void *out, int64_t rows, int64_t cols,
+                            void *stream);
+
+/* c[m, n] = *scale * sum_k x[m, k] * T[n, k] + bias[n], float32, with x split into three bf16
+ * planes that hold it exactly (products exact, float32 sums).  workspace (16-byte aligned):
+ * t81_hip_qat_matmul_workspace_size bytes; 0 there: the shape is not taken (EINVAL_SHAPE).
+ * Replaces: the F.linear of t81/nn/linear.py:93-99 and its input gradient (with the
+ * transposed limbs). */
+int64_t t81_hip_qat_matmul_workspace_size(int64_t m, int64_t n, int64_t k);
+int t81_hip_qat_matmul(const float *x, const uint8_t *w, float *c, int64_t m, int64_t n,
+                       int64_t k, const float *scale, const float *bias, void *workspace,
+                       int64_t workspace_bytes, void *stream);
+
 /* Host-only test hook, no device needed: writes the 16 x 27 tryte-contribution
  * table K4 uses (constant-evaluated like build_tryte_contributions,
  * include/t81/linalg/gemm.hpp:28-41), so it can be compared bit for bit. */

@@ -69,6 +69,11 @@ EXPORTS = (
     "t81_hip_spmm_plan_info",
     "t81_hip_spmm_plan_destroy",
     "t81_hip_spmm_simple",
+    "t81_hip_qat_scale",
+    "t81_hip_qat_quantize",
+    "t81_hip_qat_weight_grad",
+    "t81_hip_qat_matmul_workspace_size",
+    "t81_hip_qat_matmul",
     "t81_hip_limb_tryte_table",
 )
 
@@ -164,6 +169,16 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.t81_hip_spmm_plan_destroy.argtypes = [_vp]
     lib.t81_hip_spmm_simple.restype = _i
     lib.t81_hip_spmm_simple.argtypes = [_vp, _vp, _vp, _i64, _i, _i, _vp, _vp, _i, _f, _f, _vp]
+    lib.t81_hip_qat_scale.restype = _i
+    lib.t81_hip_qat_scale.argtypes = [_vp, _i, _i64, _vp, _vp, _vp, _vp]
+    lib.t81_hip_qat_quantize.restype = _i
+    lib.t81_hip_qat_quantize.argtypes = [_vp, _i, _vp, _f, _vp, _vp, _vp, _i64, _i64, _vp]
+    lib.t81_hip_qat_weight_grad.restype = _i
+    lib.t81_hip_qat_weight_grad.argtypes = [_vp, _i, _vp, _vp, _vp, _i64, _i64, _vp]
+    lib.t81_hip_qat_matmul_workspace_size.restype = _i64
+    lib.t81_hip_qat_matmul_workspace_size.argtypes = [_i64, _i64, _i64]
+    lib.t81_hip_qat_matmul.restype = _i
+    lib.t81_hip_qat_matmul.argtypes = [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp]
     lib.t81_hip_limb_tryte_table.restype = None
     lib.t81_hip_limb_tryte_table.argtypes = [_vp]
 

@@ -671,6 +671,98 @@ int t81_hip_spmm_simple(const int64_t *values, const int32_t *row_idx, const int
     return T81_HIP_OK;
 }
 
+int t81_hip_qat_scale(const void *w, int w_dtype, int64_t count, const float *previous,
+                      float *scale, void *scratch, void *stream) {
+    if (count <= 0 || too_many(count, 1))
+        return fail(T81_HIP_EINVAL_SHAPE, "the scale of a weight needs 1 to 2^40 values");
+    if (!float_dtype(w_dtype)) return fail(T81_HIP_EINVAL_DTYPE, "weights must be a float dtype");
+    if (w == nullptr || scale == nullptr || scratch == nullptr)
+        return fail(T81_HIP_EINVAL_POINTER, "null data pointer");
+    if (reinterpret_cast<uintptr_t>(w) % (w_dtype == T81_DTYPE_F32 ? 4 : 2) != 0 ||
+        reinterpret_cast<uintptr_t>(scale) % 4 != 0 ||
+        reinterpret_cast<uintptr_t>(previous) % 4 != 0 ||
+        reinterpret_cast<uintptr_t>(scratch) % 4 != 0)
+        return fail(T81_HIP_EINVAL_POINTER, "misaligned pointer");
+    if (int rc = require_device("t81_hip_qat_scale")) return rc;
+    return finish(t81hip::launch_qat_scale(w, w_dtype, count, previous, scale,
+                                           static_cast<uint32_t *>(scratch),
+                                           static_cast<hipStream_t>(stream)),
+                  "t81_hip_qat_scale");
+}
+
+// rows x cols of a float dtype: sizes whose grids of 256 threads x 12 values stay in range
+static int check_qat(int dtype, int64_t rows, int64_t cols,
+                     std::initializer_list<const void *> ptrs) {
+    if (rows < 0 || cols < 0)
+        return fail(T81_HIP_EINVAL_SHAPE, "rows and cols must be non-negative");
+    if (too_many(rows, cols) || too_many(rows, cols / 48 + 1))
+        return fail(T81_HIP_EINVAL_SHAPE, "rows x cols too large");
+    if (!float_dtype(dtype)) return fail(T81_HIP_EINVAL_DTYPE, "weights must be a float dtype");
+    if (rows > 0 && cols > 0)
+        for (const void *p : ptrs)
+            if (p == nullptr) return fail(T81_HIP_EINVAL_POINTER, "null data pointer");
+    return T81_HIP_OK;
+}
+
+int t81_hip_qat_quantize(const void *w, int w_dtype, const float *scale, float threshold,
+                         void *wq, uint8_t *packed, uint16_t *inner, int64_t rows, int64_t cols,
+                         void *stream) {
+    if (!(threshold >= 0.0f && threshold <= 1.0f))
+        return fail(T81_HIP_EINVAL_THRESHOLD, "threshold must be between 0 and 1");
+    if (int rc = check_qat(w_dtype, rows, cols, {w, scale, wq, packed, inner})) return rc;
+    const uintptr_t elem = w_dtype == T81_DTYPE_F32 ? 4 : 2;
+    if (reinterpret_cast<uintptr_t>(w) % elem != 0 || reinterpret_cast<uintptr_t>(wq) % elem != 0 ||
+        reinterpret_cast<uintptr_t>(scale) % 4 != 0 ||
+        reinterpret_cast<uintptr_t>(packed) % 4 != 0 || reinterpret_cast<uintptr_t>(inner) % 2 != 0)
+        return fail(T81_HIP_EINVAL_POINTER, "misaligned pointer");
+    if (int rc = require_device("t81_hip_qat_quantize")) return rc;
+    return finish(t81hip::launch_qat_quantize(w, w_dtype, scale, threshold, wq, packed, inner, rows,
+                                              cols, static_cast<hipStream_t>(stream)),
+                  "t81_hip_qat_quantize");
+}
+
+int t81_hip_qat_weight_grad(const void *g, int g_dtype, const float *scale,
+                            const uint16_t *inner, void *out, int64_t rows, int64_t cols,
+                            void *stream) {
+    if (int rc = check_qat(g_dtype, rows, cols, {g, scale, inner, out})) return rc;
+    const uintptr_t elem = g_dtype == T81_DTYPE_F32 ? 4 : 2;
+    if (reinterpret_cast<uintptr_t>(g) % elem != 0 || reinterpret_cast<uintptr_t>(out) % elem != 0 ||
+        reinterpret_cast<uintptr_t>(scale) % 4 != 0 || reinterpret_cast<uintptr_t>(inner) % 2 != 0)
+        return fail(T81_HIP_EINVAL_POINTER, "misaligned pointer");
+    if (int rc = require_device("t81_hip_qat_weight_grad")) return rc;
+    return finish(t81hip::launch_qat_weight_grad(g, g_dtype, scale, inner, out, rows, cols,
+                                                 static_cast<hipStream_t>(stream)),
+                  "t81_hip_qat_weight_grad");
+}
+
+int64_t t81_hip_qat_matmul_workspace_size(int64_t m, int64_t n, int64_t k) {
+    if (m <= 0 || n <= 0 || k <= 0 || m > INT_MAX / 2 || n > (int64_t(1) << 40) ||
+        k > (int64_t(1) << 31))
+        return 0;
+    return t81hip::gemm_exact_workspace_bytes(m, n, k);
+}
+
+int t81_hip_qat_matmul(const float *x, const uint8_t *w, float *c, int64_t m, int64_t n,
+                       int64_t k, const float *scale, const float *bias, void *workspace,
+                       int64_t workspace_bytes, void *stream) {
+    if (int rc = check_matmul(x, T81_DTYPE_F32, w, c, m, n, k, 1.0f, 0.0f, bias)) return rc;
+    if (m == 0 || n == 0) {
+        g_last_error.clear();
+        return T81_HIP_OK;
+    }
+    const int64_t need = t81_hip_qat_matmul_workspace_size(m, n, k);
+    if (need == 0) return fail(T81_HIP_EINVAL_SHAPE, "qat_matmul does not take this shape");
+    if (scale == nullptr || workspace == nullptr || workspace_bytes < need)
+        return fail(T81_HIP_EINVAL_POINTER, "qat_matmul needs a scale and its workspace");
+    if (reinterpret_cast<uintptr_t>(scale) % 4 != 0 ||
+        reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
+        return fail(T81_HIP_EINVAL_POINTER, "misaligned scale or workspace pointer");
+    if (int rc = require_device("t81_hip_qat_matmul")) return rc;
+    return finish(t81hip::launch_gemm_exact(x, w, c, m, n, k, scale, bias,
+                                            static_cast<hipStream_t>(stream), workspace),
+                  "t81_hip_qat_matmul");
+}
+
 void t81_hip_limb_tryte_table(double *out) { t81hip::host_tryte_table(out); }
 
 }  // extern "C"

@@ -126,7 +126,8 @@ template <int P, int CB, bool kBeta>
 __global__ __launch_bounds__(256) void gemm_planes_kernel(
     const uint8_t *__restrict__ xp, int64_t xp_bytes, const uint8_t *__restrict__ w,
     float *__restrict__ c, int M, int N, int pitch, int L, int K8, float alpha, float beta,
-    const float *__restrict__ bias, int sps, int nsplit, float *__restrict__ part) {
+    const float *__restrict__ bias, int sps, int nsplit, float *__restrict__ part,
+    const float *__restrict__ scale) {
     constexpr int RB = 4;
     constexpr int NCH = 3 * P * CB;             // chunks per half step
     constexpr int kFrags = 3 * P * CB;          // 1 KB fragments per tile
@@ -162,6 +163,7 @@ __global__ __launch_bounds__(256) void gemm_planes_kernel(
     const int grid = static_cast<int>(gridDim.x);
     const int b = static_cast<int>(blockIdx.x);
     const int pos = grid % 8 == 0 ? (b & 7) * (grid >> 3) + (b >> 3) : b;
+    if (scale != nullptr) alpha *= *scale;
     lut_fill(lut, tid, 256);  // published by the first item's barrier
 
     for (int q = pos; q < total; q += grid) {
@@ -474,7 +476,9 @@ __global__ __launch_bounds__(256) void planes_sum_kernel(const float *__restrict
                                                          float *__restrict__ c, int64_t M,
                                                          int64_t N, int nsplit, float alpha,
                                                          float beta,
-                                                         const float *__restrict__ bias) {
+                                                         const float *__restrict__ bias,
+                                                         const float *__restrict__ scale) {
+    if (scale != nullptr) alpha *= *scale;
     constexpr int V = kVec ? 4 : 1;
     const int64_t total = M * N;
     for (int64_t g = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * V; g < total;
@@ -523,6 +527,8 @@ __global__ __launch_bounds__(256) void planes_sum_kernel(const float *__restrict
 // no-allocation entry's static scratch): tokens run in chunks, or K in parts, each part's
 // product added to C.
 constexpr int64_t kPlanesWsBytes = int64_t{64} << 20;
+// three planes serve training, whose workspace comes from the caller's allocator
+constexpr int64_t planes_ws_limit(int P) { return P == 3 ? int64_t{512} << 20 : kPlanesWsBytes; }
 
 struct PlanesPlan {
     int cb = 0;                   // 32-token blocks per tile (4 or 2); 0: not taken
@@ -541,9 +547,9 @@ int64_t planes_part_offset(int P, int64_t rows, int64_t k) {
 // each its half steps plus an epilogue; a split's partials are written by the epilogues and
 // read once (5.5 TB/s).  A half step of 128 tokens took 2.05 us and of 64 tokens 1.09 us at
 // P = 2 (14336 -> 4096, M = 2048: 256 items of 150 half steps 314 us, of 300 narrow ones
-// 334 us), 1.0 / 0.72 at P = 1.
+// 334 us), 1.0 / 0.72 at P = 1, 1.6 (64 tokens) at P = 3.
 float planes_cost(int P, int cb, int64_t tiles, int64_t ns, int64_t sps, int64_t rows, int64_t n) {
-    const float step = cb == 4 ? (P == 1 ? 1.0f : 2.05f) : (P == 1 ? 0.72f : 1.09f);
+    const float step = cb == 4 ? (P == 1 ? 1.0f : 2.05f) : (P == 1 ? 0.72f : (P == 2 ? 1.09f : 1.6f));
     const int64_t cus = cu_count();
     const float rounds = static_cast<float>((tiles * ns + cus - 1) / cus);
     float t = 4.0f + rounds * (2.0f * sps * step + (cb == 4 ? 6.0f : 4.0f));
@@ -556,24 +562,25 @@ float planes_cost(int P, int cb, int64_t tiles, int64_t ns, int64_t sps, int64_t
 // (14336 -> 4096 at M = 2048: two chunks 488 us, two parts 394).
 PlanesPlan planes_plan(int P, int64_t m, int64_t n, int64_t k) {
     PlanesPlan best;
+    const int64_t limit = planes_ws_limit(P);
     const int64_t L = (k + kTrits - 1) / kTrits;
     const int64_t all_pairs = (L + 1) / 2;
-    if (m <= 0 || n <= 0 || k <= 0 || 32 * planes_image_bytes(P, 1, k) > kPlanesWsBytes ||
+    if (m <= 0 || n <= 0 || k <= 0 || 32 * planes_image_bytes(P, 1, k) > limit ||
         n >= (int64_t{1} << 30) || m >= (int64_t{1} << 30) ||
         int64_t{kPRows} * L * kTrytes >= 0x7FFFFFFF)
         return best;
     const int64_t tiles_n = (n + kPRows - 1) / kPRows;
     const int64_t cus = cu_count();
     float best_t = 0.0f;
-    const int64_t max_parts = planes_image_bytes(P, m, k) > kPlanesWsBytes ? 4 : 1;
+    const int64_t max_parts = planes_image_bytes(P, m, k) > limit ? 4 : 1;
     for (int64_t np = 1; np <= max_parts; ++np) {
         const int64_t pairs = (all_pairs + np - 1) / np;
         const int64_t parts = (all_pairs + pairs - 1) / pairs;
         const int64_t kp = parts == 1 ? k : 2 * kTrits * pairs;
         const int64_t per_tok = planes_image_bytes(P, 1, kp);
-        for (int cb = 4; cb >= 2; cb -= 2) {
+        for (int cb = P == 3 ? 2 : 4; cb >= 2; cb -= 2) {
             for (int fill = 0; fill <= 3; ++fill) {
-                int64_t count = (m * per_tok + kPlanesWsBytes - 1) / kPlanesWsBytes;
+                int64_t count = (m * per_tok + limit - 1) / limit;
                 for (int tries = 0; tries < 4; ++tries, ++count) {
                     const int64_t rows = (m + count - 1) / count;
                     const int64_t tiles = tiles_n * ((rows + 32 * cb - 1) / (32 * cb));
@@ -589,7 +596,7 @@ PlanesPlan planes_plan(int P, int64_t m, int64_t n, int64_t k) {
                     const int64_t bytes = ns > 1
                                               ? planes_part_offset(P, rows, kp) + ns * rows * n * 4
                                               : planes_image_bytes(P, rows, kp);
-                    if (bytes > kPlanesWsBytes) continue;
+                    if (bytes > limit) continue;
                     float t = planes_cost(P, cb, tiles, ns, sps, rows, n) * (count * parts);
                     // C read and written again by every part after the first
                     t += static_cast<float>((parts - 1) * m * n) * (8.0f / 4e6f);
@@ -615,7 +622,7 @@ PlanesPlan planes_plan(int P, int64_t m, int64_t n, int64_t k) {
 template <int P>
 hipError_t launch_planes(const void *x, const uint8_t *w, float *c, int64_t m, int64_t n,
                          int64_t k, float alpha, float beta, const float *bias, hipStream_t s,
-                         void *ws) {
+                         void *ws, const float *scale = nullptr) {
     using XT = std::conditional_t<P == 1, __bf16, float>;
     const PlanesPlan plan = planes_plan(P, m, n, k);
     const int64_t L = (k + kTrits - 1) / kTrits;
@@ -651,15 +658,16 @@ hipError_t launch_planes(const void *x, const uint8_t *w, float *c, int64_t m, i
             const int64_t cus = cu_count();
             const dim3 grid(static_cast<unsigned>(items < cus ? items : cus));
             const bool add = be != 0.0f && ns == 1;  // (a split's sum applies beta)
-            auto kernel = plan.cb == 4 ? (add ? gemm_planes_kernel<P, 4, true>
-                                              : gemm_planes_kernel<P, 4, false>)
-                                       : (add ? gemm_planes_kernel<P, 2, true>
-                                              : gemm_planes_kernel<P, 2, false>);
+            auto kernel = add ? gemm_planes_kernel<P, 2, true> : gemm_planes_kernel<P, 2, false>;
+            if constexpr (P != 3) {
+                if (plan.cb == 4)
+                    kernel = add ? gemm_planes_kernel<P, 4, true> : gemm_planes_kernel<P, 4, false>;
+            }
             kernel<<<grid, dim3(256), 0, s>>>(
                 image, planes_image_bytes(P, rows, kn), w + l0 * kTrytes, cc,
                 static_cast<int>(rows), static_cast<int>(n), static_cast<int>(L),
                 static_cast<int>(ln), K8, alpha, be, bi, static_cast<int>(plan.sps),
-                static_cast<int>(ns), part);
+                static_cast<int>(ns), part, scale);
             e = hipGetLastError();
             if (e != hipSuccess) return e;
             if (ns == 1) continue;
@@ -668,7 +676,7 @@ hipError_t launch_planes(const void *x, const uint8_t *w, float *c, int64_t m, i
             const int64_t blocks = (threads + 255) / 256 < 8192 ? (threads + 255) / 256 : 8192;
             auto sum = v4 ? planes_sum_kernel<true> : planes_sum_kernel<false>;
             sum<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s>>>(
-                part, cc, rows, n, static_cast<int>(ns), alpha, be, bi);
+                part, cc, rows, n, static_cast<int>(ns), alpha, be, bi, scale);
             e = hipGetLastError();
             if (e != hipSuccess) return e;
         }
@@ -700,6 +708,18 @@ hipError_t launch_gemm_planes(const float *x, const uint8_t *w, float *c, int64_
                               int64_t k, float alpha, float beta, const float *bias,
                               hipStream_t s, void *ws) {
     return launch_planes<2>(x, w, c, m, n, k, alpha, beta, bias, s, ws);
+}
+
+// Training's product: three planes (x exactly) and a scale in device memory,
+//   C[m, n] = *scale * sum_k X[m, k] * T[n, k] + bias[n].
+int64_t gemm_exact_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+    return planes_plan(3, m, n, k).bytes;
+}
+
+hipError_t launch_gemm_exact(const float *x, const uint8_t *w, float *c, int64_t m, int64_t n,
+                             int64_t k, const float *scale, const float *bias, hipStream_t s,
+                             void *ws) {
+    return launch_planes<3>(x, w, c, m, n, k, 1.0f, 0.0f, bias, s, ws, scale);
 }
 
 }  // namespace t81hip

@@ -115,6 +115,23 @@ hipError_t launch_gemm_planes(const float *x, const uint8_t *w, float *c, int64_
                               int64_t k, float alpha, float beta, const float *bias,
                               hipStream_t s, void *ws);
 
+// The same with three planes (x = hi + mid + lo exactly) and a scale in device memory, for
+// training: C = *scale * X T^T + bias.
+int64_t gemm_exact_workspace_bytes(int64_t m, int64_t n, int64_t k);
+hipError_t launch_gemm_exact(const float *x, const uint8_t *w, float *c, int64_t m, int64_t n,
+                             int64_t k, const float *scale, const float *bias, hipStream_t s,
+                             void *ws);
+
+// qat.hip (training's weight passes; dtype float32, bf16 or fp16).  scratch: 1024 words.
+hipError_t launch_qat_scale(const void *w, int dtype, int64_t count, const float *previous,
+                            float *scale, uint32_t *scratch, hipStream_t s);
+hipError_t launch_qat_quantize(const void *w, int dtype, const float *scale, float thr, void *wq,
+                               uint8_t *packed, uint16_t *inner, int64_t rows, int64_t cols,
+                               hipStream_t s);
+hipError_t launch_qat_weight_grad(const void *g, int dtype, const float *scale,
+                                  const uint16_t *inner, void *out, int64_t rows, int64_t cols,
+                                  hipStream_t s);
+
 // gemm_i8.hip (K3, int8 activations, integer matrix cores): whether a shape takes it, the
 // workspace its split-K plan uses, and the launch (C int32; accumulate: C += product)
 bool gemm_i8_fits(const void *x, int64_t m, int64_t n, int64_t k);

@@ -8,8 +8,9 @@ as in the reference).  Train mode keeps the reference's quantization-aware
 forward, ``F.linear(x, ternary(w / s) * s, b)`` with ``s`` an EMA(0.99) of max |w|
 (t81/nn/linear.py:72-99): the weight gradient flows through the dorso_round
 surrogate of :func:`t81lib_amd.qat.ternary`, and ``configure_qat`` switches on
-stochastic ternarization (t81/nn/linear.py:124-125, t81/qat.py:12-25).  Training
-is plain torch code.
+stochastic ternarization (t81/nn/linear.py:124-125, t81/qat.py:12-25).  On the GPU the
+deterministic form runs on the training kernels of :mod:`t81lib_amd.qat`; elsewhere
+training is plain torch code.
 """
 
 from __future__ import annotations
@@ -21,6 +22,7 @@ import torch
 from torch import nn
 from torch.nn import functional as F
 
+from . import qat
 from .qat import ternary
 from .tensor import TernaryTensor
 
@@ -42,7 +44,7 @@ class Linear(nn.Linear):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.training:
-            return F.linear(x, self._quantize_training_weight(), self.bias)
+            return self._training_linear(x)
         if self.ternary_weight is None:
             self.ternary_weight = TernaryTensor.from_float(
                 self.weight.detach(), threshold=self.ternary_threshold, semantics=self.semantics)
@@ -62,6 +64,18 @@ class Linear(nn.Linear):
             return out + bias if bias is not None else out
         return self.ternary_weight.linear(x, bias=bias.detach() if bias is not None else None)
 
+    def _training_linear(self, x: torch.Tensor) -> torch.Tensor:
+        if self._stochastic_rounding or \
+                type(self)._quantize_training_weight is not Linear._quantize_training_weight or \
+                not qat.weight_on_kernels(self.weight, self.ternary_threshold):
+            return F.linear(x, self._quantize_training_weight(), self.bias)
+        scale = self._update_training_scale()
+        wq, packed = qat.TernaryWeight.apply(self.weight, scale, self.ternary_threshold)
+        if not qat.product_on_kernels(x, self.weight, self.bias):
+            return F.linear(x, wq, self.bias)
+        out = qat.TernaryProduct.apply(x.reshape(-1, x.shape[-1]), wq, self.bias, packed, scale)
+        return out.reshape(*x.shape[:-1], out.shape[-1])
+
     def _quantize_training_weight(self) -> torch.Tensor:
         scale = self._update_training_scale()
         quantized = ternary(self.weight / scale, threshold=self.ternary_threshold,
@@ -69,6 +83,10 @@ class Linear(nn.Linear):
         return quantized * scale
 
     def _update_training_scale(self) -> torch.Tensor:
+        if qat.weight_on_kernels(self.weight, self.ternary_threshold) and \
+                qat.scale_on_kernels(self.training_scale):
+            self.training_scale = qat.training_scale(self.weight, self.training_scale)
+            return self.training_scale
         candidate = self.weight.detach().abs().amax().clamp(min=1e-6).to(torch.float32)
         existing = self.training_scale
         if existing is None or existing.device != candidate.device:

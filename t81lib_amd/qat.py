@@ -9,13 +9,25 @@ with |x| >= threshold take sign(x), the rest 0; with ``stochastic=True`` each su
 entry is kept with probability (|x| - threshold) / (1 - threshold) (clamped to
 [0, 1], the denominator floored at 1e-6), drawing one ``torch.rand_like`` sample
 per entry from torch's global generator -- the same draw as the reference, so a
-seeded run repeats.  Plain torch code (training runs on whatever device the
-weights are on); the packed GPU kernels serve the eval path.
+seeded run repeats.  Plain torch code, on whatever device the tensors are on.
+
+``TernaryWeight`` and ``TernaryProduct`` are the same expression, ``F.linear(x,
+ternary(w / s) * s, b)``, for ``t8.nn.Linear``'s training step on the GPU (csrc/qat.hip): the
+weight and its gradient take one pass each instead of about twenty-five, and a float32
+product runs over the packed trits with the activations split into three bf16 planes
+that hold them exactly.  Results keep the tensor expression's roundings (weights and
+weight-gradient passes bit for bit); ``weight_on_kernels`` and ``product_on_kernels`` say when
+they stand in, everything else (other devices, subclasses, tracing, forward-mode) runs the
+expression itself.
 """
 
 from __future__ import annotations
 
+from typing import Optional
+
 import torch
+
+from . import _lib, ops
 
 
 def _clamp_threshold(threshold: float) -> float:
@@ -57,6 +69,147 @@ def ternary(x: torch.Tensor, threshold: float = 0.45, stochastic: bool = False) 
     """Balanced-ternary quantization of ``x`` for training (t81/qat.py:49-57)."""
     threshold = _clamp_threshold(threshold)
     return _SurrogateGradient.apply(dorso_round(x), quantize(x, threshold, stochastic))
+
+
+# ------------------------------------------------------------- the kernels' training step --
+
+def _plain(*tensors: Optional[torch.Tensor]) -> bool:
+    """Ordinary contiguous tensors on the current GPU, outside tracing and forward-mode."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return False
+    if torch.autograd.forward_ad._current_level >= 0:
+        return False
+    for t in tensors:
+        if t is None:
+            continue
+        if type(t) not in (torch.Tensor, torch.nn.Parameter) or t.device.type != "cuda" or \
+                t.layout != torch.strided or not t.is_contiguous():
+            return False
+        if t.device.index != torch.cuda.current_device():
+            return False
+    return True
+
+
+def weight_on_kernels(weight: torch.Tensor, threshold: float) -> bool:
+    return (_plain(weight) and weight.ndim == 2 and weight.numel() > 0 and
+            weight.dtype in ops._FLOAT_CODES and threshold == threshold)
+
+
+# tokens x inputs x outputs from which the three-plane products are taken: a step of 512 x 4096
+# -> 4096 went 451 -> 343 us, 1623 x 1015 -> 3520 454 -> 344; 256 x 4096 -> 4096 stayed at
+# 286, and below that both are bound by the host, whose calls cost 30 us more (128 x 4096 ->
+# 4096 251 -> 282).
+MIN_PRODUCT = 1 << 32
+
+
+def product_on_kernels(x: torch.Tensor, weight: torch.Tensor,
+                       bias: Optional[torch.Tensor]) -> bool:
+    """Large float32 products (MIN_PRODUCT); autocast changes F.linear's own type."""
+    return (_plain(x, bias) and x.ndim >= 2 and x.dtype == torch.float32 and
+            weight.dtype == torch.float32 and x.shape[-1] == weight.shape[1] and
+            x.numel() > 0 and x.numel() * weight.shape[0] >= MIN_PRODUCT and
+            (bias is None or (bias.dtype == torch.float32 and bias.shape == weight.shape[:1])) and
+            not torch.is_autocast_enabled("cuda") and
+            _workspace(x.numel() // weight.shape[1], *weight.shape) > 0 and
+            _workspace(x.numel() // weight.shape[1], weight.shape[1], weight.shape[0]) > 0)
+
+
+def scale_on_kernels(existing: Optional[torch.Tensor]) -> bool:
+    return existing is None or (_plain(existing) and existing.ndim == 0 and
+                                existing.dtype == torch.float32 and not existing.requires_grad)
+
+
+def training_scale(weight: torch.Tensor, previous: Optional[torch.Tensor]) -> torch.Tensor:
+    """max |w| (at least 1e-6), or the 0.99 / 0.01 mean of it and the previous scale
+    (t81/nn/linear.py:72-85)."""
+    w = weight.detach()
+    scale = torch.empty((), dtype=torch.float32, device=w.device)
+    scratch = torch.empty(1024, dtype=torch.int32, device=w.device)
+    _lib.check(_lib.lib().t81_hip_qat_scale(
+        w.data_ptr(), ops._FLOAT_CODES[w.dtype], w.numel(),
+        previous.data_ptr() if previous is not None else None, scale.data_ptr(),
+        scratch.data_ptr(), ops._stream()))
+    return scale
+
+
+def _workspace(m: int, n: int, k: int) -> int:
+    return int(_lib.lib().t81_hip_qat_matmul_workspace_size(m, n, k))
+
+
+def _matmul(x: torch.Tensor, packed: torch.Tensor, n: int, scale: torch.Tensor,
+            bias: Optional[torch.Tensor]) -> torch.Tensor:
+    m, k = x.shape
+    out = torch.empty((m, n), dtype=torch.float32, device=x.device)
+    need = _workspace(m, n, k)
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+    _lib.check(_lib.lib().t81_hip_qat_matmul(
+        x.data_ptr(), packed.data_ptr(), out.data_ptr(), m, n, k, scale.data_ptr(),
+        bias.data_ptr() if bias is not None else None, ws.data_ptr(), need, ops._stream()))
+    return out
+
+
+class TernaryWeight(torch.autograd.Function):
+    """(weight, scale, threshold) -> ternary(weight / scale) * scale and its packed trits."""
+
+    @staticmethod
+    def forward(ctx, weight: torch.Tensor, scale: torch.Tensor, threshold: float):
+        rows, cols = weight.shape
+        limbs = ops.limbs_for(cols)
+        wq = torch.empty_like(weight)
+        packed = torch.empty((rows, limbs, 16), dtype=torch.uint8, device=weight.device)
+        inner = torch.empty((rows, limbs, 4), dtype=torch.uint16, device=weight.device)
+        code = ops._FLOAT_CODES[weight.dtype]
+        _lib.check(_lib.lib().t81_hip_qat_quantize(
+            weight.data_ptr(), code, scale.data_ptr(), _clamp_threshold(threshold), wq.data_ptr(),
+            packed.data_ptr(), inner.data_ptr(), rows, cols, ops._stream()))
+        ctx.save_for_backward(scale, inner)
+        ctx.mark_non_differentiable(packed)
+        ctx.set_materialize_grads(False)  # no zeros for packed
+        return wq, packed
+
+    @staticmethod
+    def backward(ctx, grad: torch.Tensor, _packed):
+        if grad is None:
+            return None, None, None
+        scale, inner = ctx.saved_tensors
+        rows, cols = grad.shape
+        if torch.is_grad_enabled() or not _plain(grad):  # a graph of the gradient is wanted
+            shifts = torch.arange(12, device=grad.device, dtype=torch.int32)
+            mask = (inner.to(torch.int32).unsqueeze(-1) >> shifts) & 1
+            mask = mask.reshape(rows, -1)[:, :cols] != 0
+            kept = torch.where(mask, grad * scale, torch.zeros_like(grad))
+            return kept * 2.0 / scale, None, None
+        out = torch.empty_like(grad)
+        _lib.check(_lib.lib().t81_hip_qat_weight_grad(
+            grad.data_ptr(), ops._FLOAT_CODES[grad.dtype], scale.data_ptr(), inner.data_ptr(),
+            out.data_ptr(), rows, cols, ops._stream()))
+        return out, None, None
+
+
+class TernaryProduct(torch.autograd.Function):
+    """F.linear(x, wq, bias) for 2-D float32 x, with wq = scale * (the packed trits)."""
+
+    @staticmethod
+    def forward(ctx, x: torch.Tensor, wq: torch.Tensor, bias: Optional[torch.Tensor],
+                packed: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
+        ctx.save_for_backward(x, wq, packed, scale)
+        return _matmul(x, packed, wq.shape[0], scale, bias)
+
+    @staticmethod
+    def backward(ctx, grad: torch.Tensor):
+        x, wq, packed, scale = ctx.saved_tensors
+        need_x, need_w, need_b = ctx.needs_input_grad[:3]
+        n, k = wq.shape
+        dx = None
+        if need_x:
+            grad_c = grad.contiguous()
+            if torch.is_grad_enabled() or not _plain(grad_c):  # a graph of the gradient is wanted
+                dx = grad @ wq
+            else:
+                dx = _matmul(grad_c, ops.transpose_packed(packed, n, k), k, scale, None)
+        dw = grad.t() @ x if need_w else None
+        db = grad.sum(0) if need_b else None
+        return dx, dw, db, None, None
 
 
 __all__ = ["ternary", "dorso_round", "quantize"]
