@@ -117,7 +117,9 @@ int t81_hip_ternary_matmul_kernel(int which, const void *x, int x_dtype, const u
  * the partials in split order (deterministic).  With float32 activations past 32 tokens the
  * workspace holds the activations' bf16 hi and lo planes (chunk by chunk of the tokens, or
  * part by part of K, where they are large) and such partials, and one launch per chunk
- * sums both planes' products.  NULL / 0 bytes: no split, no planes.  The workspace must be
+ * sums both planes' products; with bf16 ones it holds an image of them the same way where K
+ * is not a multiple of 8 or a split does not fill the CUs.  NULL / 0 bytes: no split, no
+ * planes.  The workspace must be
  * 16-byte aligned and not used by another call at the same time.
  * Replaces: the same reference interfaces as t81_hip_ternary_matmul; the
  *           reference's CPU path needs no workspace, so it has no such argument. */

@@ -1321,6 +1321,36 @@ hipError_t launch_gemm_t(const void *x, const uint8_t *w, void *c, int64_t m, in
     return hipGetLastError();
 }
 
+// bf16 activations through their image (gemm_planes.hip, one plane) instead of straight from
+// x.  The image costs a pass over x, and its product takes any K and x, in 64-token tiles
+// too.  Taken
+//  * where K is no multiple of 8 (element loads into the eight-wave kernel otherwise): 4095 ->
+//    14336 at 2048 tokens 774 -> 212 us, at 48 47 -> 26; 1003 -> 1001 at 128 26 -> 21; not
+//    where three launches cost more than that kernel (17..32 tokens 13-22 us, 4097 -> 4096 at
+//    24 14.5 -> 17.1; 511 -> 700 at 65 15.9 -> 17.0);
+//  * where the split of K over tall tiles does not fit the CUs: few tokens (4096 -> 6144 at
+//    65 / 128 / 256 30.4 -> 23.1 / 30.8 -> 25.2 / 35.6 -> 31.6 us, 14336 -> 4096 at 100
+//    56.6 -> 35.0), items past a round (3072 -> 9216 at 1024, 288 items, 90.2 -> 74.3) or far
+//    below one (8192 -> 1024 at 512 39.5 -> 30.1).  Where it fits, the split is faster
+//    (14336 -> 4096 at 512 68 -> 86, 4096 -> 6144 at 512 43 -> 52), as it is over fewer than
+//    2 Mi weights (1088 -> 1639 at 96 18.7 -> 20.7) and, past 128 tokens, where C takes no
+//    16-byte stores (8768 -> 6781 at 148 46.9 -> 54.7).
+bool gemm_use_plane(int64_t m, int64_t n, int64_t k) {
+    if (k % 8 != 0) {
+        const int64_t weights = n < (int64_t{1} << 30) ? n * k : int64_t{1} << 62;
+        if (m <= 16) return false;
+        if (m <= 32) return weights >= int64_t{1} << 25;
+        return m >= 96 || weights >= int64_t{1} << 20;
+    }
+    if (m <= 64 || gemm_rows_whole_rounds(m, n) != 0 || n * k < (int64_t{1} << 21)) return false;
+    if (m <= 128) return true;
+    if (n % 4 != 0) return false;
+    const SplitPlan p = gemm_split_plan_tall(m, n, k);
+    const int64_t cus = cu_count();
+    return p.nsplit * p.tiles > cus || (m <= 256 && p.nsplit >= 4) ||
+           (m <= 1024 && 5 * p.nsplit * p.tiles < 3 * cus);
+}
+
 template <int XT>
 hipError_t launch_gemm_x(const void *x, const uint8_t *w, void *c, int64_t m, int64_t n,
                          int64_t k, float alpha, float beta, const float *bias, hipStream_t s,
@@ -1332,6 +1362,12 @@ hipError_t launch_gemm_x(const void *x, const uint8_t *w, void *c, int64_t m, in
         if (planes > 0 && ws != nullptr && ws_bytes >= planes)
             return launch_gemm_planes(static_cast<const float *>(x), w, static_cast<float *>(c), m,
                                       n, k, alpha, beta, bias, s, ws);
+    }
+    if constexpr (XT == kDtypeBF16) {
+        const int64_t plane = gemm_use_plane(m, n, k) ? gemm_plane_workspace_bytes(m, n, k) : 0;
+        if (plane > 0 && ws != nullptr && ws_bytes >= plane)
+            return launch_gemm_plane(x, w, static_cast<float *>(c), m, n, k, alpha, beta, bias, s,
+                                     ws);
     }
     if constexpr (XT == kDtypeBF16 || XT == kDtypeI8) {
         // 17..64 tokens, aligned: the column-block stream kernel of K2 (gemv.hip)
@@ -1494,6 +1530,12 @@ int64_t gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, int x_dtype) {
     if (m <= 0 || n <= 0 || k <= 0) return 0;
     switch (x_dtype) {
         case kDtypeBF16:
+            if (gemm_use_plane(m, n, k)) {
+                // (not less than the split's, so a size never shrinks with the path taken)
+                const int64_t plane = gemm_plane_workspace_bytes(m, n, k);
+                const int64_t split = gemm_workspace_x<kDtypeBF16>(m, n, k);
+                if (plane > 0) return plane > split ? plane : split;
+            }
             // the column-block stream kernel's shapes (17..gemv_column_blocks_max_tokens
             // tokens, K % 8 == 0): no workspace
             if (m >= 17 && m <= gemv_column_blocks_max_tokens(k, x_dtype) && k % 8 == 0)

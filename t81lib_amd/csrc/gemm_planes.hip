@@ -1,10 +1,9 @@
-// t81lib_amd/csrc/gemm_planes.hip -- K3 for float32 activations: one launch over their
-// bf16 planes.
+// t81lib_amd/csrc/gemm_planes.hip -- K3 through an image of the activations' bf16 planes.
 //
 //   C[m, n] = alpha * sum_k X[m, k] * T[n, k] + beta * C[m, n] + bias[n]
 //
-// x is cut into P bf16 planes (P = 2: hi + lo, |x - hi - lo| <= 2^-18 |x|) by a first
-// small kernel, and the product kernel accumulates every plane's products into the same
+// x is cut into P bf16 planes (P = 2: float32 as hi + lo, |x - hi - lo| <= 2^-18 |x|; P = 3:
+// float32 exactly; P = 1: bf16 as it is) by a first small kernel, and the product kernel accumulates every plane's products into the same
 // accumulators: each decoded weight fragment meets P planes before it is dropped, so the
 // trit decode and the weight loads per MFMA are 1 / P of the bf16 kernel's.  What bounds it
 // is the matrix pipe (2 P M N K flops).
@@ -708,6 +707,16 @@ hipError_t launch_gemm_planes(const float *x, const uint8_t *w, float *c, int64_
                               int64_t k, float alpha, float beta, const float *bias,
                               hipStream_t s, void *ws) {
     return launch_planes<2>(x, w, c, m, n, k, alpha, beta, bias, s, ws);
+}
+
+int64_t gemm_plane_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+    return planes_plan(1, m, n, k).bytes;
+}
+
+hipError_t launch_gemm_plane(const void *x, const uint8_t *w, float *c, int64_t m, int64_t n,
+                             int64_t k, float alpha, float beta, const float *bias,
+                             hipStream_t s, void *ws) {
+    return launch_planes<1>(x, w, c, m, n, k, alpha, beta, bias, s, ws);
 }
 
 // Training's product: three planes (x exactly) and a scale in device memory,

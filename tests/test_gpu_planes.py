@@ -44,3 +44,32 @@ def test_planes_keep_tokens_apart(gpu):
     rest = [m for m in range(M) if m not in (3, 69)]
     assert torch.equal(y[rest], clean[rest])
     assert torch.isnan(y[69]).all() and not torch.isfinite(y[3]).any()
+
+
+# bf16 activations through their image: K that is no multiple of 8 (and x off alignment), few
+# tokens over a split that does not fit, tokens and rows past a tile, one limb pair
+BF16 = [(17, 8193, 4100, 0), (33, 1025, 1030, 0), (96, 97, 513, 1), (130, 1001, 512, 0),
+        (100, 4096, 1030, 0), (129, 2048, 2052, 0), (200, 4096, 1536, 3), (65, 4104, 600, 0)]
+
+
+@pytest.mark.parametrize("M,K,N,offset", BF16)
+def test_bf16_image_bit_exact(gpu, orc, M, K, N, offset):
+    """Integer activations |x| <= 127: every partial sum is an integer below 2^24."""
+    announce(f"bf16 image M={M} K={K} N={N} offset={offset}")
+    g = torch.Generator("cpu").manual_seed(M + K + N)
+    packed = ops.quantize_pack(torch.randn((N, K), generator=g).to(gpu), 0.45, _lib.THR_CPP)
+    xi = torch.randint(-127, 128, (M, K), generator=g)
+    store = torch.zeros(M * K + 8, dtype=torch.bfloat16, device=gpu)
+    x = store[offset:offset + M * K].view(M, K)
+    x.copy_(xi.to(gpu))
+    acc = torch.from_numpy(orc.trit_matmul_i64(xi.to(torch.int8).numpy(), packed.cpu().numpy(), K))
+    c = torch.randint(-1000, 1001, (M, N), generator=g).float()
+    bias = torch.randint(-1000, 1001, (N,), generator=g).float()
+    for alpha, beta, use_bias in ((1.0, 0.0, False), (0.5, 1.0, True)):
+        out = ops.ternary_matmul(x, packed, K, alpha=alpha, beta=beta,
+                                 c=c.to(gpu) if beta else None,
+                                 bias=bias.to(gpu) if use_bias else None)
+        want = alpha * acc.double() + (beta * c.double() if beta else 0.0)
+        if use_bias:
+            want = want + bias.double()
+        assert torch.equal(out.cpu().double(), want), f"alpha={alpha}"
