@@ -365,6 +365,12 @@ int t81_hip_qat_matmul(const float *x, const uint8_t *w, float *c, int64_t m, in
                        int64_t k, const float *scale, const float *bias, void *workspace,
                        int64_t workspace_bytes, void *stream);
 
+/* out[c] = sum over rows of g[r, c] (rows x cols float32, row-major), the gradient of a bias;
+ * fixed order.  scratch: t81_hip_column_sum_scratch_size bytes (0: none needed). */
+int64_t t81_hip_column_sum_scratch_size(int64_t rows, int64_t cols);
+int t81_hip_column_sum(const float *g, float *out, int64_t rows, int64_t cols, void *scratch,
+                       int64_t scratch_bytes, void *stream);
+
 /* Host-only test hook, no device needed: writes the 16 x 27 tryte-contribution
  * table K4 uses (constant-evaluated like build_tryte_contributions,
  * include/t81/linalg/gemm.hpp:28-41), so it can be compared bit for bit. */

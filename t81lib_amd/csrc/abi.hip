@@ -763,6 +763,30 @@ int t81_hip_qat_matmul(const float *x, const uint8_t *w, float *c, int64_t m, in
                   "t81_hip_qat_matmul");
 }
 
+int64_t t81_hip_column_sum_scratch_size(int64_t rows, int64_t cols) {
+    if (rows < 0 || cols < 0 || too_many(rows, cols)) return 0;
+    return t81hip::column_sum_scratch_bytes(rows, cols);
+}
+
+int t81_hip_column_sum(const float *g, float *out, int64_t rows, int64_t cols, void *scratch,
+                       int64_t scratch_bytes, void *stream) {
+    if (rows < 0 || cols < 0)
+        return fail(T81_HIP_EINVAL_SHAPE, "rows and cols must be non-negative");
+    if (too_many(rows, cols)) return fail(T81_HIP_EINVAL_SHAPE, "rows x cols too large");
+    if (cols > 0 && (out == nullptr || (rows > 0 && g == nullptr)))
+        return fail(T81_HIP_EINVAL_POINTER, "null data pointer");
+    const int64_t need = t81_hip_column_sum_scratch_size(rows, cols);
+    if (need > 0 && (scratch == nullptr || scratch_bytes < need))
+        return fail(T81_HIP_EINVAL_POINTER, "column_sum needs its scratch");
+    if (reinterpret_cast<uintptr_t>(g) % 4 != 0 || reinterpret_cast<uintptr_t>(out) % 4 != 0 ||
+        reinterpret_cast<uintptr_t>(scratch) % 4 != 0)
+        return fail(T81_HIP_EINVAL_POINTER, "misaligned pointer");
+    if (int rc = require_device("t81_hip_column_sum")) return rc;
+    return finish(t81hip::launch_column_sum(g, out, rows, cols, static_cast<float *>(scratch),
+                                            static_cast<hipStream_t>(stream)),
+                  "t81_hip_column_sum");
+}
+
 void t81_hip_limb_tryte_table(double *out) { t81hip::host_tryte_table(out); }
 
 }  // extern "C"

@@ -222,6 +222,75 @@ __global__ __launch_bounds__(256) void qat_weight_grad_kernel(
     store12<T, kVec>(out + r * cols, c0, cols, v);
 }
 
+// Column sums of a row-major float32 matrix.  A block of four waves takes 256 columns (64: V =
+// 1) of a run of rows, wave w rows w, w + 4, ... with four loads in flight, and adds its waves'
+// sums; the runs' sums are added in order by a second kernel.  (1024 x 14336: tensor sum 53
+// us, the two kernels 17.)
+template <int V>
+__global__ __launch_bounds__(256) void column_sum_kernel(const float *__restrict__ g,
+                                                         float *__restrict__ out, int64_t rows,
+                                                         int64_t cols, int64_t run) {
+    __shared__ float part[4][64 * V];
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int64_t c = (static_cast<int64_t>(blockIdx.x) * 64 + lane) * V;
+    const int64_t r0 = static_cast<int64_t>(blockIdx.y) * run;
+    const int64_t r1 = r0 + run < rows ? r0 + run : rows;
+    float acc[4][V] = {};
+    auto load = [&](int64_t r, float (&v)[V]) {
+        if constexpr (V == 4) {
+            const f32x4 x = *reinterpret_cast<const f32x4 *>(g + r * cols + c);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = x[u];
+        } else {
+            v[0] = g[r * cols + c];
+        }
+    };
+    if (c < cols) {
+        int64_t r = r0 + wave;
+        for (; r + 12 < r1; r += 16) {
+            float v[4][V];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) load(r + 4 * i, v[i]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int u = 0; u < V; ++u) acc[i][u] += v[i][u];
+        }
+        for (; r < r1; r += 4) {
+            float v[V];
+            load(r, v);
+#pragma unroll
+            for (int u = 0; u < V; ++u) acc[0][u] += v[u];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < V; ++u)
+        part[wave][lane * V + u] = (acc[0][u] + acc[1][u]) + (acc[2][u] + acc[3][u]);
+    __syncthreads();
+    for (int i = threadIdx.x; i < 64 * V; i += 256) {
+        const int64_t col = static_cast<int64_t>(blockIdx.x) * 64 * V + i;
+        if (col < cols)
+            out[blockIdx.y * cols + col] = (part[0][i] + part[1][i]) + (part[2][i] + part[3][i]);
+    }
+}
+
+__global__ __launch_bounds__(256) void column_sum_runs_kernel(const float *__restrict__ part,
+                                                              float *__restrict__ out,
+                                                              int64_t cols, int runs) {
+    const int64_t c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (c >= cols) return;
+    float a = 0.0f;
+    for (int r = 0; r < runs; r += 8) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = r + i < runs ? part[(r + i) * cols + c] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a += v[i];
+    }
+    out[c] = a;
+}
+
 int64_t blocks_for(int64_t n) { return (n + 255) / 256; }
 
 template <typename T>
@@ -267,6 +336,35 @@ hipError_t qat_weight_grad_t(const void *g, const float *scale, const uint16_t *
 }
 
 }  // namespace
+
+// Rows per run: 64, more once there would be over 64 runs.
+static int64_t column_sum_run(int64_t rows) {
+    const int64_t run = (rows + 63) / 64;
+    return run < 64 ? 64 : (run + 15) / 16 * 16;
+}
+
+int64_t column_sum_scratch_bytes(int64_t rows, int64_t cols) {
+    const int64_t runs = (rows + column_sum_run(rows) - 1) / column_sum_run(rows);
+    return runs > 1 ? runs * cols * 4 : 0;
+}
+
+hipError_t launch_column_sum(const float *g, float *out, int64_t rows, int64_t cols,
+                             float *scratch, hipStream_t s) {
+    if (cols == 0) return hipSuccess;
+    const int64_t run = column_sum_run(rows);
+    const int64_t runs = rows > 0 ? (rows + run - 1) / run : 1;
+    float *part = runs > 1 ? scratch : out;
+    const bool vec = cols % 4 == 0 && reinterpret_cast<uintptr_t>(g) % 16 == 0;
+    const int64_t wide = vec ? 256 : 64;
+    const dim3 grid(static_cast<unsigned>((cols + wide - 1) / wide), static_cast<unsigned>(runs));
+    auto kernel = vec ? column_sum_kernel<4> : column_sum_kernel<1>;
+    kernel<<<grid, dim3(256), 0, s>>>(g, part, rows, cols, run);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || runs == 1) return e;
+    column_sum_runs_kernel<<<dim3(static_cast<unsigned>(blocks_for(cols))), dim3(256), 0, s>>>(
+        part, out, cols, static_cast<int>(runs));
+    return hipGetLastError();
+}
 
 hipError_t launch_qat_scale(const void *w, int dtype, int64_t count, const float *previous,
                             float *scale, uint32_t *scratch, hipStream_t s) {

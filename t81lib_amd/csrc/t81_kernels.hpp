@@ -137,6 +137,11 @@ hipError_t launch_qat_weight_grad(const void *g, int dtype, const float *scale,
                                   const uint16_t *inner, void *out, int64_t rows, int64_t cols,
                                   hipStream_t s);
 
+// Column sums of a rows x cols float32 matrix; scratch of column_sum_scratch_bytes.
+int64_t column_sum_scratch_bytes(int64_t rows, int64_t cols);
+hipError_t launch_column_sum(const float *g, float *out, int64_t rows, int64_t cols,
+                             float *scratch, hipStream_t s);
+
 // gemm_i8.hip (K3, int8 activations, integer matrix cores): whether a shape takes it, the
 // workspace its split-K plan uses, and the launch (C int32; accumulate: C += product)
 bool gemm_i8_fits(const void *x, int64_t m, int64_t n, int64_t k);

@@ -24,7 +24,7 @@ from torch.nn import functional as F
 
 from . import qat
 from .qat import ternary
-from .tensor import TernaryTensor
+from .tensor import TernaryTensor, _linear_under_grad
 
 _DEFAULT_THRESHOLD = 0.45
 
@@ -59,9 +59,8 @@ class Linear(nn.Linear):
             raise ValueError("t81.nn.Linear expects 2D or 3D inputs")
         bias = self.bias
         if torch.is_grad_enabled() and (x.requires_grad or (bias is not None and bias.requires_grad)):
-            # autograd: dx through the transposed limbs, dbias through the addition
-            out = self.ternary_weight.matmul_input(x)
-            return out + bias if bias is not None else out
+            # autograd: dx through the transposed limbs, dbias as column sums
+            return _linear_under_grad(self.ternary_weight, x, bias)
         return self.ternary_weight.linear(x, bias=bias.detach() if bias is not None else None)
 
     def _training_linear(self, x: torch.Tensor) -> torch.Tensor:

@@ -230,6 +230,23 @@ def ternary_matmul(x: torch.Tensor, w_packed: torch.Tensor, k: Optional[int] = N
     return c
 
 
+def column_sum(g: torch.Tensor) -> torch.Tensor:
+    """Sums over the rows of a 2-D float32 GPU tensor (the gradient of a bias)."""
+    _require_cuda(g, "g")
+    if g.ndim != 2 or g.dtype != torch.float32:
+        raise ValueError("column_sum expects a 2D float32 tensor")
+    g = g.contiguous()
+    rows, cols = g.shape
+    out = torch.empty(cols, dtype=torch.float32, device=g.device)
+    lib = _lib.lib()
+    need = int(lib.t81_hip_column_sum_scratch_size(rows, cols))
+    scratch = torch.empty(need, dtype=torch.uint8, device=g.device) if need else None
+    _lib.check(lib.t81_hip_column_sum(g.data_ptr(), out.data_ptr(), rows, cols,
+                                      scratch.data_ptr() if scratch is not None else None, need,
+                                      _stream()))
+    return out
+
+
 def gemm_limb(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, m: int, n: int, k: int,
               alpha: float = 1.0, beta: float = 0.0) -> torch.Tensor:
     """K4: the reference's limb-integer gemm_ternary, C updated in place.
@@ -267,7 +284,7 @@ def limb_tryte_table() -> "list[list[float]]":
 
 __all__ = [
     "quantize_pack", "quantize", "pack_cols", "unpack", "count_invalid_bytes", "ternary_matmul",
-    "gemm_limb", "limb_tryte_table", "limbs_for", "torch_threshold",
+    "column_sum", "gemm_limb", "limb_tryte_table", "limbs_for", "torch_threshold",
 ]
 
 

@@ -208,7 +208,9 @@ class TernaryProduct(torch.autograd.Function):
             else:
                 dx = _matmul(grad_c, ops.transpose_packed(packed, n, k), k, scale, None)
         dw = grad.t() @ x if need_w else None
-        db = grad.sum(0) if need_b else None
+        db = None
+        if need_b:
+            db = grad.sum(0) if torch.is_grad_enabled() or not _plain(grad) else ops.column_sum(grad)
         return dx, dw, db, None, None
 
 

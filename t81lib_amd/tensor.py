@@ -247,6 +247,46 @@ class _TernaryGemmFunction(torch.autograd.Function):
         return None, grad_rhs
 
 
+class _TernaryLinearFunction(torch.autograd.Function):
+    """x @ T^T + bias for x (tokens, cols) with the bias in the kernel's epilogue; backward dx
+    over the transposed limbs, dbias as column sums (the same values as _TernaryGemmFunction
+    and an addition, without a pass over the output and its gradient's tensor sum)."""
+
+    @staticmethod
+    def forward(ctx, ternary_weight: TernaryTensor, x: torch.Tensor,
+                bias: Optional[torch.Tensor]) -> torch.Tensor:
+        ctx.ternary = ternary_weight
+        return ops.ternary_matmul(_activations(x), ternary_weight._packed,
+                                  ternary_weight._k_actual, bias=bias)
+
+    @staticmethod
+    def backward(ctx, grad_output: torch.Tensor):
+        t: TernaryTensor = ctx.ternary
+        g = grad_output.contiguous()
+        dx = db = None
+        if ctx.needs_input_grad[1]:
+            dx = ops.ternary_matmul(g, t.transposed_packed(), t._rows)
+        if ctx.needs_input_grad[2]:
+            # (a graph of the gradient, where one is wanted, comes from the tensor sum)
+            db = g.sum(0) if torch.is_grad_enabled() else ops.column_sum(g)
+        return None, dx, db
+
+
+def _linear_under_grad(ternary: TernaryTensor, x: torch.Tensor,
+                       bias: Optional[torch.Tensor]) -> torch.Tensor:
+    """x (tokens, cols) @ T^T + bias recorded for autograd."""
+    if (ternary._semantics == "trit_dot" and type(x) in (torch.Tensor, nn.Parameter) and
+            x.is_floating_point() and x.dtype != torch.float64 and x.device.type == "cuda" and
+            x.ndim == 2 and x.shape[1] == ternary._k_actual and
+            (bias is None or (type(bias) in (torch.Tensor, nn.Parameter) and
+                              bias.shape == (ternary._rows,) and bias.device == x.device and
+                              bias.dtype in (torch.float32, torch.bfloat16, torch.float16))) and
+            torch.autograd.forward_ad._current_level < 0):
+        return _TernaryLinearFunction.apply(ternary, x, bias)
+    out = ternary.matmul_input(x)
+    return out + bias if bias is not None else out
+
+
 # ------------------------------------------------- whole-network conversion --
 # Semantics given to the TernaryTensors that model.to(dtype=trit) creates.
 conversion_semantics = "trit_dot"
@@ -343,9 +383,7 @@ def _ternary_linear_forward(self: nn.Linear, input: torch.Tensor) -> torch.Tenso
     grad = torch.is_grad_enabled() and (
         input.requires_grad or (bias is not None and bias.requires_grad))
     if grad or x.device.type != "cuda" or ternary._semantics != "trit_dot":
-        out = ternary.matmul_input(x)
-        if bias is not None:
-            out = out + bias
+        out = _linear_under_grad(ternary, x, bias)
     else:
         out = ternary.linear(x, bias=bias.detach() if bias is not None else None)
     return out.reshape(*lead, out.shape[-1]) if input.ndim != 2 else out
