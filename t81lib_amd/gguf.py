@@ -19,6 +19,7 @@ from typing import Optional, Sequence
 import torch
 
 from . import _lib
+from .ops import _stream
 
 GGML_TYPE_TQ1_0 = _lib.TQ1_0  # t81/gguf.py:30
 GGML_TYPE_TQ2_0 = _lib.TQ2_0  # t81/gguf.py:31
@@ -34,10 +35,6 @@ def _quant_code(quant: "str | int") -> int:
     if isinstance(quant, str) and quant.upper() in _QUANTS:
         return _QUANTS[quant.upper()]
     raise ValueError(f"quant must be one of {sorted(_QUANTS)}")
-
-
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
 
 
 def row_bytes(cols: int, quant: "str | int") -> int:

@@ -21,12 +21,9 @@ import numpy as np
 import torch
 
 from . import _lib
+from .ops import _stream
 
 INT32_MIN, INT32_MAX = -2**31, 2**31 - 1
-
-
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
 
 
 def entry_arrays(values: Any, row_indices: Any, col_indices: Any,

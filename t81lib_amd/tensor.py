@@ -205,7 +205,7 @@ class TernaryTensor(torch.Tensor):
 
 
 def _activations(x: torch.Tensor) -> torch.Tensor:
-    if x.device.type != "cuda":
+    if not x.is_cuda:
         raise ValueError("activations must be on the GPU")
     if x.dtype not in (torch.float32, torch.bfloat16, torch.int8):
         x = x.float()
