@@ -14,9 +14,11 @@
 //   (v * 256 + 242) / 243, so digit n reads back as ((uint8)(byte * 3^n) * 3) >> 8.
 // All float arithmetic is float32 with separate roundings (no contraction), as numpy
 // evaluates it.  Rows are zero-padded to whole blocks.  Dequantize writes with the
-// non-temporal hint (every output byte is written once); whole-block rows into an
+// non-temporal hint (every output byte is written once); rows of whole float4s into an
 // aligned output as one float4 per lane.
 #include <hip/hip_fp16.h>
+
+#include <type_traits>
 
 #include "t81_device.hpp"
 #include "t81_kernels.hpp"
@@ -44,6 +46,14 @@ __device__ __forceinline__ int tq_trit(float v, int use_thr, float thr) {
     return static_cast<int>(r);
 }
 
+// Row of block b with nb blocks per row (a 64-bit division is a long sequence: 1.7 us of the
+// dequantize's 17 at 8192 x 3072).
+__device__ __forceinline__ int64_t block_row(int64_t b, int64_t nb) {
+    if (((b | nb) >> 32) == 0)
+        return static_cast<uint32_t>(b) / static_cast<uint32_t>(nb);
+    return b / nb;
+}
+
 // Max over the wavefront (lane values >= 0 or NaN-free by construction).
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
@@ -51,74 +61,124 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-// Whole blocks of a 16-byte aligned matrix (cols a multiple of 256): lane l reads values
-// 4 l .. 4 l + 3 of its wavefront's block with one non-temporal float4 (each value is read
-// once), takes the block max from those, turns them into digits (trit + 1) and writes the
-// four digits to the wavefront's 256-byte LDS slot; each lane then gathers the digits its
-// output byte packs, in the layouts described at the top.  The slot is private to the
-// wavefront, whose LDS operations complete in order, so no barrier is needed.
-// (8192 x 3072: TQ1_0 63.5 -> 26.1 us, TQ2_0 57.7 -> 24.3 against tq_quantize_kernel.)
-template <int Q>
+// Max of max(v, the value `ctrl` brings from another lane), without LDS.
+template <int ctrl, int rows = 0xF>
+__device__ __forceinline__ float dpp_max(float v) {
+    const int o = __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), ctrl, rows, 0xF,
+                                              false);
+    return fmaxf(v, __int_as_float(o));
+}
+__device__ __forceinline__ float wave_max_dpp(float v) {
+    v = dpp_max<0xB1>(v);         // quad_perm 1 0 3 2
+    v = dpp_max<0x4E>(v);         // quad_perm 2 3 0 1
+    v = dpp_max<0x141>(v);        // row_half_mirror
+    v = dpp_max<0x140>(v);        // row_mirror: every lane holds its row's max
+    v = dpp_max<0x142, 0xA>(v);   // row_bcast 15 into rows 1 and 3
+    v = dpp_max<0x143, 0xC>(v);   // row_bcast 31 into rows 2 and 3: lane 63 holds all
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+// B = 4 consecutive blocks per wavefront (2 below 8192 blocks, where few wavefronts are in
+// flight).  HBM-bound (4 bytes read per weight): B 16-byte loads are in flight per lane, and
+// the rest is kept off their way.  Lane l holds weights
+// 4 l .. 4 l + 3 of each block and writes their digits (trit + 1) as one dword to the
+// wavefront's LDS slot; since a base-3 number of five digits stays below 243 and two-bit
+// fields do not meet, an output dword (four bytes) is then formed from 4 or 5 such dwords
+// with no carry between its bytes: 13 lanes (TQ1_0) or 16 (TQ2_0) per block, all the blocks
+// at once.  Their payload bytes are contiguous and go out as dwords through
+// LDS.  kVec: rows are 16-byte aligned runs of whole float4s, else element loads; columns past
+// the row are zeros.  The slots are private to the wavefront, whose LDS operations complete
+// in order, so no barrier is needed.  8192 x 3072: TQ1_0 28.3 -> 23.1 us, TQ2_0 25.3 ->
+// 20.5 against one block per wavefront with byte gathers; 8192 x 3008 (partial blocks) 62.7
+// -> 21.4, 8191 x 3071 64.3 -> 28.8 against strided loads read twice.
+template <int Q, bool kVec, int B>
 __global__ __launch_bounds__(256) void tq_quantize_vec_kernel(const float *__restrict__ src,
                                                               uint8_t *__restrict__ dst,
-                                                              int64_t blocks, float thr,
+                                                              int64_t blocks, int64_t cols,
+                                                              int64_t nb, float thr,
                                                               int use_thr) {
-    __shared__ uint32_t slots[4][64];
+    static_assert(B % 2 == 0, "a wavefront's payload is whole dwords");
+    constexpr int kDw = Q == kTq1 ? 13 : 16;           // digit dwords per block
+    constexpr int kHalves = tq_bytes(Q) / 2;           // 16-bit words per block
+    __shared__ uint32_t slots[4][B * 64];
+    __shared__ __attribute__((aligned(4))) uint16_t outs[4][B * kHalves];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t blk = static_cast<int64_t>(blockIdx.x) * 4 + wave;
-    if (blk >= blocks) return;  // whole wavefront
-    const floatx4 x =
-        __builtin_nontemporal_load(reinterpret_cast<const floatx4 *>(src + blk * kQK) + lane);
-    float mx = 0.0f;
-    bool nan = false;
+    const int64_t blk0 = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * B;
+    if (blk0 >= blocks) return;  // whole wavefront
+    const int n = blocks - blk0 < B ? static_cast<int>(blocks - blk0) : B;
+    floatx4 x[B];
+    int64_t r = block_row(blk0, nb), cb = blk0 - r * nb;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const float a = fabsf(x[u]);
-        nan |= a != a;
-        mx = fmaxf(mx, a);
-    }
-    mx = wave_max(mx);
-    const float d = __builtin_amdgcn_ballot_w64(nan) != 0 ? __builtin_nanf("") : mx;
-    const float inv_d = d == 0.0f ? 0.0f : 1.0f / d;
-    uint32_t dig = 0;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-        dig |= static_cast<uint32_t>(tq_trit(x[u] * inv_d, use_thr, thr) + 1) << (8 * u);
-    slots[wave][lane] = dig;
-    __builtin_amdgcn_wave_barrier();
-    const uint8_t *sd = reinterpret_cast<const uint8_t *>(slots[wave]);
-    uint8_t *out = dst + blk * tq_bytes(Q);
-    if constexpr (Q == kTq2) {
-        const int a = lane >> 5;
-        const int c = lane & 31;
-        uint32_t b = 0;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) b |= static_cast<uint32_t>(sd[a * 128 + s * 32 + c]) << (2 * s);
-        out[lane] = static_cast<uint8_t>(b);
-    } else {
-        if (lane < 52) {
-            int first, stride, ndig;
-            if (lane < 32) {
-                first = lane, stride = 32, ndig = 5;
-            } else if (lane < 48) {
-                first = 160 + (lane - 32), stride = 16, ndig = 5;
+    for (int u = 0; u < B; ++u) {
+        x[u] = floatx4{0.f, 0.f, 0.f, 0.f};
+        const int64_t col = cb * kQK + 4 * lane;
+        const float *p = src + r * cols + col;
+        if (u < n) {
+            if constexpr (kVec) {
+                if (col < cols) x[u] = __builtin_nontemporal_load(reinterpret_cast<const floatx4 *>(p));
             } else {
-                first = 240 + (lane - 48), stride = 4, ndig = 4;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (col + j < cols) x[u][j] = p[j];
             }
+        }
+        if (++cb == nb) cb = 0, ++r;
+    }
+    uint16_t *out = outs[wave];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+        float mx = 0.0f;
+        bool nan = false;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float a = fabsf(x[u][j]);
+            nan |= a != a;
+            mx = fmaxf(mx, a);
+        }
+        mx = wave_max_dpp(mx);
+        const float d = __builtin_amdgcn_ballot_w64(nan) != 0 ? __builtin_nanf("") : mx;
+        const float inv_d = d == 0.0f ? 0.0f : 1.0f / d;
+        uint32_t dig = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            dig |= static_cast<uint32_t>(tq_trit(x[u][j] * inv_d, use_thr, thr) + 1) << (8 * j);
+        slots[wave][64 * u + lane] = dig;
+        if (lane == u) out[kHalves * (u + 1) - 1] = __half_as_ushort(__float2half_rn(d));
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (lane < B * kDw) {
+        const int u = lane / kDw, o = lane - u * kDw;
+        const uint32_t *sd = slots[wave] + 64 * u;
+        uint32_t b = 0;
+        if constexpr (Q == kTq2) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) b |= sd[32 * (o >> 3) + 8 * s + (o & 7)] << (2 * s);
+        } else {
+            // dwords 0-7: five digits 32 weights apart; 8-11: 16 apart from 160; 12: four
+            // digits 4 apart from 240, weighted 81, 27, 9, 3
+            const int first = o < 8 ? o : (o < 12 ? 40 + (o - 8) : 60);
+            const int step = o < 8 ? 8 : (o < 12 ? 4 : 1);
             uint32_t v = 0;
 #pragma unroll
-            for (int i = 0; i < 5; ++i)
-                if (i < ndig) v = v * 3 + sd[first + i * stride];
-            if (ndig == 4) v *= 3;  // four digits weighted 81, 27, 9, 3
-            out[lane] = static_cast<uint8_t>((v * 256u + 242u) / 243u);
+            for (int i = 0; i < 4; ++i) v = v * 3u + sd[first + i * step];
+            v = v * 3u + (o < 12 ? sd[first + 4 * step] : 0u);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                b |= ((((v >> (8 * j)) & 0xFFu) * 256u + 242u) / 243u) << (8 * j);
         }
+        out[kHalves * u + 2 * o] = static_cast<uint16_t>(b);
+        out[kHalves * u + 2 * o + 1] = static_cast<uint16_t>(b >> 16);
     }
-    if (lane == 0) {
-        const uint16_t h = __half_as_ushort(__float2half_rn(d));
-        out[tq_bytes(Q) - 2] = static_cast<uint8_t>(h & 0xFFu);
-        out[tq_bytes(Q) - 1] = static_cast<uint8_t>(h >> 8);
-    }
+    __builtin_amdgcn_wave_barrier();
+    // blk0 is a multiple of B and two blocks are whole dwords: dst + blk0 tq_bytes is 4-byte
+    // aligned where dst is
+    const uint32_t *words = reinterpret_cast<const uint32_t *>(out);
+    uint32_t *g = reinterpret_cast<uint32_t *>(dst + blk0 * tq_bytes(Q));
+    const int halves = n * kHalves;
+    for (int i = lane; i < halves / 2; i += 64) g[i] = words[i];
+    if (halves % 2 != 0 && lane == 0)
+        reinterpret_cast<uint16_t *>(g)[halves - 1] = out[halves - 1];
 }
 
 template <int Q>
@@ -187,62 +247,18 @@ __global__ __launch_bounds__(256) void tq_quantize_kernel(const float *__restric
     }
 }
 
-template <int Q>
-__global__ __launch_bounds__(256) void tq_dequantize_kernel(const uint8_t *__restrict__ src,
-                                                            float *__restrict__ dst,
-                                                            int64_t rows, int64_t cols,
-                                                            int64_t nb) {
-    const int lane = threadIdx.x & 63;
-    const int64_t blk =
-        static_cast<int64_t>(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (blk >= rows * nb) return;
-    const int64_t r = blk / nb;
-    const int64_t col0 = (blk - r * nb) * kQK;
-    const uint8_t *in = src + blk * tq_bytes(Q);
-    const uint16_t h = static_cast<uint16_t>(in[tq_bytes(Q) - 2] | (in[tq_bytes(Q) - 1] << 8));
-    const float d = __half2float(__ushort_as_half(h));
-    float *row = dst + r * cols;
-    auto put = [&](int j, int digit) {
-        const int64_t col = col0 + j;
-        if (col < cols) __builtin_nontemporal_store(d * static_cast<float>(digit - 1), row + col);
-    };
-    if constexpr (Q == kTq2) {
-        const uint32_t b = in[lane];
-        const int a = lane >> 5;
-        const int c = lane & 31;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) put(a * 128 + s * 32 + c, static_cast<int>((b >> (2 * s)) & 3u));
-    } else if (lane < 52) {
-        const uint32_t b = in[lane];
-        int first, stride, ndig;
-        if (lane < 32) {
-            first = lane, stride = 32, ndig = 5;
-        } else if (lane < 48) {
-            first = 160 + (lane - 32), stride = 16, ndig = 5;
-        } else {
-            first = 240 + (lane - 48), stride = 4, ndig = 4;
-        }
-        uint32_t p = 1;
-#pragma unroll
-        for (int n = 0; n < 5; ++n) {
-            if (n < ndig) {
-                const uint32_t q = (b * p) & 0xFFu;
-                put(first + n * stride, static_cast<int>((q * 3u) >> 8));
-            }
-            p *= 3;
-        }
-    }
-}
-
-// Whole blocks (cols a multiple of 256) into a 16-byte aligned output, where block b's
-// weights are outputs 256 b .. 256 b + 255: lane l writes weights 4 l .. 4 l + 3 with one
-// non-temporal float4.  Those four share a digit position: TQ2_0 bits 2s of four
+// One wavefront per block.  Rows of whole float4s (cols a multiple of 4) into a 16-byte aligned
+// output (kVec): lane l writes weights 4 l .. 4 l + 3 of its block with one non-temporal
+// float4, past the row none (8192 x 3008 TQ1_0 28.4 -> 16.0 us against element stores).
+// Else the block turns through LDS so that each store is 64 consecutive floats (8191 x 3071
+// TQ1_0 64.3 -> 37.0).  Those four share a digit position: TQ2_0 bits 2s of four
 // consecutive bytes; TQ1_0 digit n of four consecutive bytes (n = e / 32 below 160,
 // (e - 160) / 16 below 240, (e - 240) / 4 after, e = 4 l).
-template <int Q>
-__global__ __launch_bounds__(256) void tq_dequantize_vec_kernel(const uint8_t *__restrict__ src,
+template <int Q, bool kVec>
+__global__ __launch_bounds__(256) void tq_dequantize_kernel(const uint8_t *__restrict__ src,
                                                                 float *__restrict__ dst,
-                                                                int64_t blocks) {
+                                                                int64_t blocks, int64_t cols,
+                                                                int64_t nb) {
     const int lane = threadIdx.x & 63;
     const int64_t blk =
         static_cast<int64_t>(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -279,7 +295,27 @@ __global__ __launch_bounds__(256) void tq_dequantize_vec_kernel(const uint8_t *_
     floatx4 o;
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[j] = d * static_cast<float>(digit[j] - 1);
-    __builtin_nontemporal_store(o, reinterpret_cast<floatx4 *>(dst + blk * kQK + e));
+    if (kVec && cols == nb * kQK) {  // whole blocks: no row to find
+        __builtin_nontemporal_store(o, reinterpret_cast<floatx4 *>(dst + blk * kQK + e));
+        return;
+    }
+    const int64_t r = block_row(blk, nb);
+    const int64_t col0 = (blk - r * nb) * kQK;
+    float *row = dst + r * cols;
+    if constexpr (kVec) {
+        if (col0 + e < cols)
+            __builtin_nontemporal_store(o, reinterpret_cast<floatx4 *>(row + col0 + e));
+    } else {
+        __shared__ __attribute__((aligned(16))) float turn[4][kQK];
+        float *t = turn[threadIdx.x >> 6];
+        *reinterpret_cast<floatx4 *>(t + e) = o;
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int64_t col = col0 + 64 * j + lane;
+            if (col < cols) row[col] = t[64 * j + lane];
+        }
+    }
 }
 
 }  // namespace
@@ -289,16 +325,24 @@ hipError_t launch_tq_quantize(const float *src, uint8_t *dst, int64_t rows, int6
     const int64_t nb = (cols + kQK - 1) / kQK;
     const int64_t blocks = rows * nb;
     if (blocks == 0) return hipSuccess;
-    const dim3 grid(static_cast<unsigned>((blocks + 3) / 4));
-    if (cols % kQK == 0 && (reinterpret_cast<uintptr_t>(src) & 15u) == 0) {
-        if (quant == kTq2)
-            tq_quantize_vec_kernel<kTq2><<<grid, 256, 0, s>>>(src, dst, blocks, thr, use_thr);
-        else
-            tq_quantize_vec_kernel<kTq1><<<grid, 256, 0, s>>>(src, dst, blocks, thr, use_thr);
-    } else if (quant == kTq2)
-        tq_quantize_kernel<kTq2><<<grid, 256, 0, s>>>(src, dst, rows, cols, nb, thr, use_thr);
-    else
-        tq_quantize_kernel<kTq1><<<grid, 256, 0, s>>>(src, dst, rows, cols, nb, thr, use_thr);
+    if (reinterpret_cast<uintptr_t>(dst) % 4 != 0) {  // dword stores of the payload
+        const dim3 grid(static_cast<unsigned>((blocks + 3) / 4));
+        auto kernel = quant == kTq2 ? tq_quantize_kernel<kTq2> : tq_quantize_kernel<kTq1>;
+        kernel<<<grid, 256, 0, s>>>(src, dst, rows, cols, nb, thr, use_thr);
+        return hipGetLastError();
+    }
+    const bool vec = cols % 4 == 0 && (reinterpret_cast<uintptr_t>(src) & 15u) == 0;
+    const bool few = blocks < 8192;
+    const int64_t per = few ? 8 : 16;
+    const dim3 grid(static_cast<unsigned>((blocks + per - 1) / per));
+    auto pick = [&](auto q) {
+        constexpr int Q = decltype(q)::value;
+        if (few) return vec ? tq_quantize_vec_kernel<Q, true, 2> : tq_quantize_vec_kernel<Q, false, 2>;
+        return vec ? tq_quantize_vec_kernel<Q, true, 4> : tq_quantize_vec_kernel<Q, false, 4>;
+    };
+    auto kernel = quant == kTq2 ? pick(std::integral_constant<int, kTq2>())
+                                : pick(std::integral_constant<int, kTq1>());
+    kernel<<<grid, 256, 0, s>>>(src, dst, blocks, cols, nb, thr, use_thr);
     return hipGetLastError();
 }
 
@@ -308,16 +352,10 @@ hipError_t launch_tq_dequantize(const uint8_t *src, float *dst, int64_t rows, in
     const int64_t blocks = rows * nb;
     if (blocks == 0) return hipSuccess;
     const dim3 grid(static_cast<unsigned>((blocks + 3) / 4));
-    if (cols % kQK == 0 && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
-        if (quant == kTq2)
-            tq_dequantize_vec_kernel<kTq2><<<grid, 256, 0, s>>>(src, dst, blocks);
-        else
-            tq_dequantize_vec_kernel<kTq1><<<grid, 256, 0, s>>>(src, dst, blocks);
-    } else if (quant == kTq2) {
-        tq_dequantize_kernel<kTq2><<<grid, 256, 0, s>>>(src, dst, rows, cols, nb);
-    } else {
-        tq_dequantize_kernel<kTq1><<<grid, 256, 0, s>>>(src, dst, rows, cols, nb);
-    }
+    const bool vec = cols % 4 == 0 && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0;
+    auto kernel = quant == kTq2 ? (vec ? tq_dequantize_kernel<kTq2, true> : tq_dequantize_kernel<kTq2, false>)
+                                : (vec ? tq_dequantize_kernel<kTq1, true> : tq_dequantize_kernel<kTq1, false>);
+    kernel<<<grid, 256, 0, s>>>(src, dst, blocks, cols, nb);
     return hipGetLastError();
 }
 
