@@ -1021,6 +1021,9 @@ bool gemm_use_half(int64_t m, int64_t n, int64_t n1) {
     return n1 > 0 && n1 < n && m > 64 && t <= cus && 4 * t >= 3 * cus;
 }
 
+struct SplitPlan;
+SplitPlan gemm_split_plan_tall(int64_t m, int64_t n, int64_t k);
+
 // How the big-tile kernel splits K for a shape: with few tiles (< 160), about one
 // workgroup per CU in total, at least four k-steps per split.  nsplit == 1: no split.
 struct SplitPlan {
@@ -1044,19 +1047,27 @@ int64_t split_workspace_bytes(const SplitPlan &p) {
 }
 
 // 384 x 128 tiles (three 32-row blocks per wave, the waves along the rows: the RB = 3,
-// WR = 4 instance) when a shape has fewer 256 x 256 tiles than CUs but 160 or more (no
-// split), and its 384 x 128 tiles still fit one round: every CU then runs one tile of
-// about three quarters the work instead of three quarters of the CUs one tile each (qkv
-// at M = 2048: 192 -> 256 tiles).  The 2 x 2 form of the same tiles (192 x 256) measured
-// slower: qkv M = 2048 83.2 -> 80.7 us, with beta = 1 95.4 -> 89.8 us, 3072 -> 3072 at
-// M = 4096 66.2 -> 64.7 us, a ragged 2000 x 4104 -> 6000 95.9 -> 90.9 us.
+// WR = 4 instance) where they fit one round of the CUs:
+//  * of a shape with 160 or more 256 x 256 tiles (no split) but fewer than CUs: every CU then
+//    runs one tile of about three quarters the work instead of three quarters of the CUs one
+//    tile each (qkv at M = 2048: 192 -> 256 tiles, 83.2 -> 80.7 us, with beta = 1 95.4 -> 89.8;
+//    3072 -> 3072 at M = 4096 66.2 -> 64.7).
+//  * of a shape with fewer, up to K = 8192, instead of a split of K and its sum: from 160 of
+//    them (3072 -> 9216 at M = 777 58.7 -> 51.9 us, at 1024 90.1 -> 54.6, 4096 -> 6144 at 1300
+//    104.5 -> 66.0, 2048 -> 8192 at 1024 51.3 -> 43.2), or from half a round where the split's
+//    items run past a round of the CUs (4096 -> 6144 at 1024, 96 tall tiles x 3, 79.8 -> 66.0).
+//    Not below (4096 -> 4096 at 1700, 154 of them, 65.5 -> 69.5), nor over K = 14336, whose
+//    partials weigh less beside its steps (2048 tokens 188 -> 239).
 bool gemm_use_384(int64_t m, int64_t n, int64_t k) {
     const int64_t L = (k + kTrits - 1) / kTrits;
     const int64_t t4 = ((n + kW4Rows - 1) / kW4Rows) * ((m + kW4Tokens - 1) / kW4Tokens);
     const int64_t t3 = ((n + 383) / 384) * ((m + 127) / 128);
     const int64_t cus = cu_count();
-    return m > 64 && t4 >= 160 && t4 < cus && t3 <= cus &&
-           int64_t(384) * L * kTrytes < 0x7FFFFFFF;
+    if (m <= 64 || t4 >= cus || t3 > cus || int64_t(384) * L * kTrytes >= 0x7FFFFFFF) return false;
+    if (t4 >= 160) return true;
+    if (k > 8192 || 2 * t3 < cus) return false;
+    const SplitPlan p = gemm_split_plan_tall(m, n, k);
+    return t3 >= 160 || p.nsplit * p.tiles > cus;
 }
 hipError_t launch_gemm_w4_384(const void *x, const uint8_t *w, void *c, int64_t m, int64_t n,
                               int64_t ldc, int64_t k, float alpha, float beta, const float *bias,
@@ -1344,7 +1355,7 @@ bool gemm_use_plane(int64_t m, int64_t n, int64_t k) {
     }
     if (m <= 64 || gemm_rows_whole_rounds(m, n) != 0 || n * k < (int64_t{1} << 21)) return false;
     if (m <= 128) return true;
-    if (n % 4 != 0) return false;
+    if (n % 4 != 0 || gemm_use_384(m, n, k)) return false;
     const SplitPlan p = gemm_split_plan_tall(m, n, k);
     const int64_t cus = cu_count();
     return p.nsplit * p.tiles > cus || (m <= 256 && p.nsplit >= 4) ||

@@ -99,7 +99,8 @@ __device__ __forceinline__ void i8_lut_fill(uint8_t *lds, int tid, int nthreads)
 // WR = 4: tall 512 x 128 tiles (the four waves side by side along the rows, each still
 // 128 rows x 128 tokens; half the activation-tile loads per step), half-width 512 x 64,
 // no split-K items (their sum assumes 2 x 2 waves).
-template <bool kHalf, bool kAcc, int WR = 2>
+// RB = 3 (WR = 4): 384 x 128 tiles, three 32-row blocks per wave, whole tiles only.
+template <bool kHalf, bool kAcc, int WR = 2, int RB = 4>
 __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
     const int8_t *__restrict__ x, const uint8_t *__restrict__ w, int32_t *__restrict__ c, int M,
     int N, int ldc, int K, int L, int accumulate, int n1, int sps, i32x4 *__restrict__ part,
@@ -130,9 +131,11 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     static_assert(WR == 2 || WR == 4, "waves 2 x 2, or 4 along the rows");
+    static_assert(RB == 4 || (RB == 3 && WR == 4 && !kHalf), "384-row tiles are whole tiles");
     if constexpr (WR == 4) nsplit = 0;
+    if constexpr (RB == 3) n1 = N;
     constexpr int WT = 4 / WR;           // waves along the tokens
-    constexpr int kRowsT = 128 * WR;     // weight rows per tile
+    constexpr int kRowsT = 32 * RB * WR;  // weight rows per tile
     constexpr int kTokT = 128 * WT;      // tokens per whole tile
     const int wn = WR == 4 ? wave : wave & 1;
     const int wm = WR == 4 ? 0 : wave >> 1;
@@ -149,8 +152,8 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
     const int all_steps = (L + 1) / 2;
     i8_lut_fill(lut, tid, kI8Threads);  // published by the first item's barrier
 
-    // One item: 128 WR weight rows (nwg..) x 32 CB WT tokens (m0..) over k-steps
-    // [s_begin, s_end); wave (wn, wm) owns 128 rows x 32 CB tokens.  CB = 4: whole or
+    // One item: 32 RB WR weight rows (nwg..) x 32 CB WT tokens (m0..) over k-steps
+    // [s_begin, s_end); wave (wn, wm) owns 32 RB rows x 32 CB tokens.  CB = 4: whole or
     // split-K tiles; CB = 2: half-width tiles.
     auto run_item = [&](auto cbc, int nwg, int m0, int s_begin, int s_end, bool split, int sp,
                         int tt) {
@@ -160,14 +163,14 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
         constexpr int kTL = 32 * CB * WT * kI8RowSlots / 64;
         constexpr int LPW = (kTL + 3) / 4;
         constexpr int NCH = 3 * CB;                        // chunks of four MFMAs per step
-        constexpr int NFC = CB == 4 ? 8 : 4;               // chunks that issue table reads
-        constexpr int kWLoads = 4;                         // loads of fetch_w: one per row block
+        constexpr int NFC = RB == 3 ? 6 : (CB == 4 ? 8 : 4);  // chunks that issue table reads
+        constexpr int kWLoads = RB;                        // loads of fetch_w: one per row block
         // all but the newest fetch_w: the tile loads issued before it have landed
         constexpr int kWaitW = waitcnt_vm<kWLoads>();
         // every wave is past the previous item's epilogue (staged in the tile buffers)
         // before this item's tile loads
         __syncthreads();
-        constexpr int FR = 8 / NFC;                        // ... for FR x 2 row blocks each
+        constexpr int FR = RB == 3 ? 1 : 8 / NFC;          // ... for FR x 2 row blocks each
         // The lane index passes through an empty asm once per item (its derived offsets are
         // recomputed per item, not kept live across the epilogue).
         int lane = tid & 63;
@@ -179,15 +182,15 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
         // row's first limb or zeros -- finite trits that meet zero activations
         const __amdgpu_buffer_rsrc_t wsrc = i8_rsrc(w + static_cast<int64_t>(nwg) * L * kTrytes,
                                                     static_cast<int64_t>(N - nwg) * L * kTrytes);
-        uint32_t woff[4];
+        uint32_t woff[RB];
 #pragma unroll
-        for (int rb = 0; rb < 4; ++rb)
-            woff[rb] = (static_cast<uint32_t>(128 * wn + 32 * rb + r) * static_cast<uint32_t>(L) +
+        for (int rb = 0; rb < RB; ++rb)
+            woff[rb] = (static_cast<uint32_t>(32 * RB * wn + 32 * rb + r) * static_cast<uint32_t>(L) +
                         static_cast<uint32_t>(h)) * kTrytes;
-        auto fetch_w = [&](int step, u32x4 (&dst)[4]) {
+        auto fetch_w = [&](int step, u32x4 (&dst)[RB]) {
             const uint32_t koff = static_cast<uint32_t>(step) * (2 * kTrytes);
 #pragma unroll
-            for (int rb = 0; rb < 4; ++rb)
+            for (int rb = 0; rb < RB; ++rb)
                 dst[rb] = __builtin_bit_cast(
                     u32x4, __builtin_amdgcn_raw_buffer_load_b128(wsrc, woff[rb] + koff, 0, 0));
         };
@@ -244,9 +247,9 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
             out[2] = __builtin_amdgcn_alignbit(t[3], t[2], 16);
         };
 
-        i32x16 acc[4][CB];
+        i32x16 acc[RB][CB];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < RB; ++i)
 #pragma unroll
             for (int j = 0; j < CB; ++j)
 #pragma unroll
@@ -264,11 +267,11 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
 
         // Weights run three steps ahead: wcur holds step s, wnxt step s + 1, wn2 step s + 2
         // (loaded during step s - 1), and step s + 3 is loaded into wn3 during step s.
-        u32x4 wcur[4], wnxt[4], wn2[4], wn3[4];
-        i32x4 a[2][4][3];   // operands of the step with parity P / of the other one
+        u32x4 wcur[RB], wnxt[RB], wn2[RB], wn3[RB];
+        i32x4 a[2][RB][3];   // operands of the step with parity P / of the other one
         // merge the table words of weight dword dw of row block rb into operand dwords
         // 3 dw .. 3 dw + 2 (operand d / 4, component d % 4)
-        auto merge_into = [&](const uint32_t (&t)[4], i32x4 (&ops)[4][3], int rb, int dw) {
+        auto merge_into = [&](const uint32_t (&t)[4], i32x4 (&ops)[RB][3], int rb, int dw) {
             uint32_t o[3];
             table_merge(t, o);
 #pragma unroll
@@ -281,12 +284,15 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
         // frb(gf, e), e < FR: the first half of those chunks dwords 2 and 3 of this step
         // (the rest of its J = 1 and J = 2 operands), the second half dwords 0 and 1 of the
         // next step (its J = 0 operands and the start of its J = 1)
-        auto fdw = [&](int gf) {
-            if constexpr (CB == 4) return gf < 4 ? 2 + gf / 2 : (gf - 4) / 2;
+        // (RB = 3: two of the twelve lookups a chunk, in dword order)
+        auto fdw = [&](int gf, int e) {
+            if constexpr (RB == 3) return 2 * gf + e < 6 ? 2 + (2 * gf + e) / 3 : (2 * gf + e - 6) / 3;
+            else if constexpr (CB == 4) return gf < 4 ? 2 + gf / 2 : (gf - 4) / 2;
             else return gf < 2 ? 2 + gf : gf - 2;
         };
         auto frb = [&](int gf, int e) {
-            if constexpr (CB == 4) return 2 * (gf % 2) + e;
+            if constexpr (RB == 3) return (2 * gf + e) % 3;
+            else if constexpr (CB == 4) return 2 * (gf % 2) + e;
             else return e;
         };
 
@@ -301,7 +307,7 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
         if (s_begin < s_end) {
             // the first step's J = 0 operands and dwords 4, 5 of its J = 1 operands
 #pragma unroll
-            for (int rb = 0; rb < 4; ++rb)
+            for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
                 for (int dw = 0; dw < 2; ++dw) {
                     uint32_t t[4];
@@ -332,17 +338,17 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
                     const int gp = g - 1;
 #pragma unroll
                     for (int e = 0; e < 2 * FR; ++e) {
-                        if (gp < NFC / 2) merge_into(t[gp & 1][e], a[P], frb(gp, e), fdw(gp));
-                        else merge_into(t[gp & 1][e], a[P ^ 1], frb(gp, e), fdw(gp));
+                        if (gp < NFC / 2) merge_into(t[gp & 1][e], a[P], frb(gp, e), fdw(gp, e));
+                        else merge_into(t[gp & 1][e], a[P ^ 1], frb(gp, e), fdw(gp, e));
                     }
                 }
                 if (g < NFC) {
 #pragma unroll
                     for (int e = 0; e < 2 * FR; ++e)
-                        table_fetch((g < NFC / 2 ? wcur : wnxt)[frb(g, e)][fdw(g)], t[g & 1][e]);
+                        table_fetch((g < NFC / 2 ? wcur : wnxt)[frb(g, e)][fdw(g, e)], t[g & 1][e]);
                 }
 #pragma unroll
-                for (int rb = 0; rb < 4; ++rb)
+                for (int rb = 0; rb < RB; ++rb)
                     acc[rb][g % CB] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
                         a[P][rb][g / CB], bq[g % 3], acc[rb][g % CB], 0, 0, 0);
                 // each MFMA followed by a few of the chunk's other instructions (three LDS
@@ -351,7 +357,7 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
                 // one-tryte table; with the pair table two reads and three VALU measured the
                 // same or up to 2 % slower)
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
+                for (int k = 0; k < RB; ++k) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
                     __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // LDS read
                     __builtin_amdgcn_sched_group_barrier(0x006, 4, 0);   // VALU, SALU
@@ -360,7 +366,7 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
                 __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int rb = 0; rb < 4; ++rb) {
+            for (int rb = 0; rb < RB; ++rb) {
                 wcur[rb] = wnxt[rb];
                 wnxt[rb] = wn2[rb];
                 wn2[rb] = wn3[rb];
@@ -378,12 +384,12 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
         if (step < s_end)  // odd step count: the last step, peeled
             step_body(step, B0(), B1());
 
-        if constexpr (CB == 4) {
+        if constexpr (CB == 4 && RB == 4) {
             if (split) {
                 i32x4 *dst =
                     part + (((static_cast<int64_t>(sp) * tiles2 + tt) * 4 + wave) * 64) * 64 + lane;
 #pragma unroll
-                for (int rb = 0; rb < 4; ++rb)
+                for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
                     for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
@@ -407,11 +413,11 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
         auto c_pass = [&](int p, i32x4 (&cv)[8]) {
             const int cb = p / 2;
             const int rp = p % 2;
-            const int nb = col0 + 128 * wn + 64 * rp + tc;
+            const int nb = col0 + 32 * RB * wn + 64 * rp + tc;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int m = m0 + 32 * CB * wm + 32 * cb + 4 * i + tq;
-                const bool ok = vec4 && m < M && nb + 3 < N;
+                const bool ok = vec4 && m < M && tc < (2 * rp + 1 < RB ? 64 : 32) && nb + 3 < N;
                 // non-temporal, as the bf16 kernel's C reads (gate_up M = 2048 with C
                 // accumulated: 283.0 -> 270.9 us)
                 i32x4 t = {0, 0, 0, 0};
@@ -434,18 +440,20 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
                     if (pass + 1 < kPasses) c_pass(pass + 1, cvn);
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
+                    if (2 * rp + j < RB)
 #pragma unroll
                     for (int a4 = 0; a4 < 4; ++a4)
                         *reinterpret_cast<i32x4 *>(&st[r * kI8StageStride + 32 * j + 8 * a4 + 4 * h]) =
                             i32x4{acc[2 * rp + j][cb][4 * a4], acc[2 * rp + j][cb][4 * a4 + 1],
                                   acc[2 * rp + j][cb][4 * a4 + 2], acc[2 * rp + j][cb][4 * a4 + 3]};
-                const int nb = col0 + 128 * wn + 64 * rp + tc;
+                const int nb = col0 + 32 * RB * wn + 64 * rp + tc;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     const int tok = 4 * i + tq;
                     const i32x4 v = *reinterpret_cast<const i32x4 *>(&st[tok * kI8StageStride + tc]);
                     const int m = m0 + 32 * CB * wm + 32 * cb + tok;
-                    if (m >= M) continue;
+                    // rows of this pass: 64, or 32 for the third block of three
+                    if (m >= M || tc >= (2 * rp + 1 < RB ? 64 : 32)) continue;
                     int32_t *cr = c + static_cast<int64_t>(m) * ldc;
                     int32_t y[4] = {v[0], v[1], v[2], v[3]};
                     if (vec4 && nb + 3 < N) {
@@ -601,6 +609,19 @@ I8Plan i8_plan(int64_t m, int64_t n, int64_t k) {
     return p;
 }
 
+// 384 x 128 tiles where they are half a round of the CUs to a whole one, instead of 256 x 256
+// tiles on fewer CUs or their split of K and its int32 sum: 4096 -> 6144 at M = 1536 84.3 ->
+// 48.6 us, at 900 62.3 -> 45.4, at 2048 62.8 -> 56.6; 3072 -> 9216 at 1024 73.9 -> 39.9; 2048 ->
+// 8192 at 777 39.6 -> 32.5.  Over a K past 8192 a split that fits stays faster (14336 -> 4096 at
+// 2048 133 -> 163), so only where there is none (at 2500 tokens 197 -> 167).
+bool i8_use_384(int64_t m, int64_t n, int64_t k) {
+    const int64_t L = (k + kTrits - 1) / kTrits;
+    const int64_t t3 = ((n + 383) / 384) * ((m + 127) / 128);
+    const int64_t cus = cu_count();
+    if (t3 > cus || 2 * t3 < cus || int64_t(384) * L * kTrytes >= 0x7FFFFFFF) return false;
+    return k <= 8192 || i8_rows_whole_rounds(m, n) != 0;
+}
+
 }  // namespace
 
 // Whether the integer big-tile kernel takes this shape: more than 64 tokens, K a multiple
@@ -643,6 +664,16 @@ hipError_t launch_gemm_i8(const void *x, const uint8_t *w, int32_t *c, int64_t m
             static_cast<const int8_t *>(x), w, c, static_cast<int>(m), static_cast<int>(n),
             static_cast<int>(n), static_cast<int>(k), static_cast<int>(L), accumulate ? 1 : 0,
             static_cast<int>(tn1), 0, nullptr, 0);
+        return hipGetLastError();
+    }
+    const int64_t t384 = ((n + 383) / 384) * ((m + 127) / 128);
+    if (i8_use_384(m, n, k)) {
+        auto kernel = accumulate ? gemm_w4_i8_kernel<false, true, 4, 3>
+                                 : gemm_w4_i8_kernel<false, false, 4, 3>;
+        kernel<<<dim3(static_cast<unsigned>(t384)), dim3(kI8Threads), 0, s>>>(
+            static_cast<const int8_t *>(x), w, c, static_cast<int>(m), static_cast<int>(n),
+            static_cast<int>(n), static_cast<int>(k), static_cast<int>(L), accumulate ? 1 : 0,
+            static_cast<int>(n), 0, nullptr, 0);
         return hipGetLastError();
     }
     I8Plan p = i8_plan(m, n, k);
