@@ -365,6 +365,15 @@ int t81_hip_qat_matmul(const float *x, const uint8_t *w, float *c, int64_t m, in
                        int64_t k, const float *scale, const float *bias, void *workspace,
                        int64_t workspace_bytes, void *stream);
 
+/* c[n, k] = sum_m g[m, n] * x[m, k] (float32, row-major; the weight's gradient of that
+ * product), both operands split into three bf16 planes that hold them exactly and the six
+ * largest plane products summed in float32.  workspace (16-byte aligned):
+ * t81_hip_qat_weight_product_workspace_size bytes; 0 there: not taken (EINVAL_SHAPE). */
+int64_t t81_hip_qat_weight_product_workspace_size(int64_t m, int64_t n, int64_t k);
+int t81_hip_qat_weight_product(const float *g, const float *x, float *c, int64_t m, int64_t n,
+                               int64_t k, void *workspace, int64_t workspace_bytes,
+                               void *stream);
+
 /* out[c] = sum over rows of g[r, c] (rows x cols float32, row-major), the gradient of a bias;
  * fixed order.  scratch: t81_hip_column_sum_scratch_size bytes (0: none needed). */
 int64_t t81_hip_column_sum_scratch_size(int64_t rows, int64_t cols);

@@ -74,6 +74,8 @@ EXPORTS = (
     "t81_hip_qat_weight_grad",
     "t81_hip_qat_matmul_workspace_size",
     "t81_hip_qat_matmul",
+    "t81_hip_qat_weight_product_workspace_size",
+    "t81_hip_qat_weight_product",
     "t81_hip_column_sum_scratch_size",
     "t81_hip_column_sum",
     "t81_hip_limb_tryte_table",
@@ -181,6 +183,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.t81_hip_qat_matmul_workspace_size.argtypes = [_i64, _i64, _i64]
     lib.t81_hip_qat_matmul.restype = _i
     lib.t81_hip_qat_matmul.argtypes = [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp]
+    lib.t81_hip_qat_weight_product_workspace_size.restype = _i64
+    lib.t81_hip_qat_weight_product_workspace_size.argtypes = [_i64, _i64, _i64]
+    lib.t81_hip_qat_weight_product.restype = _i
+    lib.t81_hip_qat_weight_product.argtypes = [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp]
     lib.t81_hip_column_sum_scratch_size.restype = _i64
     lib.t81_hip_column_sum_scratch_size.argtypes = [_i64, _i64]
     lib.t81_hip_column_sum.restype = _i

@@ -23,7 +23,8 @@ ARCH = "gfx950"
 
 SOURCES = ["abi.hip", "pack.hip", "gemv.hip", "gemv_strip.hip", "gemm.hip", "gemm_planes.hip", "gemm_i8.hip",
            "limb.hip", "elementwise.hip", "tq.hip", "tq_row.hip", "gemv_tq2.hip", "transpose.hip",
-           "spmm.hip", "noalloc.hip", "qat.hip"]
+           "spmm.hip", "noalloc.hip", "qat.hip",
+           "gemm_wgrad.hip"]
 
 # -packed-fp32-ops: no v_pk_*_f32 from the compiler (they are never written by hand either).
 HIPCC_FLAGS = [

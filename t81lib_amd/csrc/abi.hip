@@ -763,6 +763,27 @@ int t81_hip_qat_matmul(const float *x, const uint8_t *w, float *c, int64_t m, in
                   "t81_hip_qat_matmul");
 }
 
+int64_t t81_hip_qat_weight_product_workspace_size(int64_t m, int64_t n, int64_t k) {
+    return t81hip::gemm_wgrad_workspace_bytes(m, n, k);
+}
+
+int t81_hip_qat_weight_product(const float *g, const float *x, float *c, int64_t m, int64_t n,
+                               int64_t k, void *workspace, int64_t workspace_bytes,
+                               void *stream) {
+    const int64_t need = t81_hip_qat_weight_product_workspace_size(m, n, k);
+    if (need == 0) return fail(T81_HIP_EINVAL_SHAPE, "qat_weight_product does not take this shape");
+    if (g == nullptr || x == nullptr || c == nullptr || workspace == nullptr ||
+        workspace_bytes < need)
+        return fail(T81_HIP_EINVAL_POINTER, "qat_weight_product needs its data and workspace");
+    if (reinterpret_cast<uintptr_t>(g) % 4 != 0 || reinterpret_cast<uintptr_t>(x) % 4 != 0 ||
+        reinterpret_cast<uintptr_t>(c) % 4 != 0 || reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
+        return fail(T81_HIP_EINVAL_POINTER, "misaligned pointer");
+    if (int rc = require_device("t81_hip_qat_weight_product")) return rc;
+    return finish(t81hip::launch_gemm_wgrad(g, x, c, m, n, k, static_cast<hipStream_t>(stream),
+                                            workspace),
+                  "t81_hip_qat_weight_product");
+}
+
 int64_t t81_hip_column_sum_scratch_size(int64_t rows, int64_t cols) {
     if (rows < 0 || cols < 0 || too_many(rows, cols)) return 0;
     return t81hip::column_sum_scratch_bytes(rows, cols);

@@ -127,6 +127,16 @@ hipError_t launch_gemm_exact(const float *x, const uint8_t *w, float *c, int64_t
                              int64_t k, const float *scale, const float *bias, hipStream_t s,
                              void *ws);
 
+// The row-major rows x cols partials part + sp rows cols, added in split order into c.
+hipError_t launch_planes_sum(const float *part, float *c, int64_t rows, int64_t cols, int nsplit,
+                             hipStream_t s);
+
+// gemm_wgrad.hip: C (n x k) = G^T X for G (m x n), X (m x k), float32; workspace bytes (0: the
+// shape is not taken).
+int64_t gemm_wgrad_workspace_bytes(int64_t m, int64_t n, int64_t k);
+hipError_t launch_gemm_wgrad(const float *g, const float *x, float *c, int64_t m, int64_t n,
+                             int64_t k, hipStream_t s, void *ws);
+
 // qat.hip (training's weight passes; dtype float32, bf16 or fp16).  scratch: 1024 words.
 hipError_t launch_qat_scale(const void *w, int dtype, int64_t count, const float *previous,
                             float *scale, uint32_t *scratch, hipStream_t s);

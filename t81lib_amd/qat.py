@@ -148,6 +148,27 @@ def _matmul(x: torch.Tensor, packed: torch.Tensor, n: int, scale: torch.Tensor,
     return out
 
 
+# outputs from which the six-plane product stands in for the float32 one: its 256 x 256 tiles
+# split the tokens below, and the library's smaller tiles are faster there (4096 tokens,
+# 1024 x 1024: 63 us against 81; 2048 x 2048 232 -> 188, 1623 tokens, 3520 x 1015 154 -> 106,
+# 2048 tokens, 4096 x 4096 479 -> 302).
+MIN_WEIGHTS = 3 << 20
+
+
+def weight_product(grad: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """grad^T @ x for contiguous float32 grad (m, n) and x (m, k)."""
+    (m, n), k = grad.shape, x.shape[1]
+    lib = _lib.lib()
+    need = lib.t81_hip_qat_weight_product_workspace_size(m, n, k) if n * k >= MIN_WEIGHTS else 0
+    if need == 0:  # (or operands whose planes pass the workspace's bound)
+        return grad.t() @ x
+    out = torch.empty((n, k), dtype=torch.float32, device=x.device)
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+    _lib.check(lib.t81_hip_qat_weight_product(grad.data_ptr(), x.data_ptr(), out.data_ptr(), m, n,
+                                              k, ws.data_ptr(), need, ops._stream()))
+    return out
+
+
 class TernaryWeight(torch.autograd.Function):
     """(weight, scale, threshold) -> ternary(weight / scale) * scale and its packed trits."""
 
@@ -200,17 +221,22 @@ class TernaryProduct(torch.autograd.Function):
         x, wq, packed, scale = ctx.saved_tensors
         need_x, need_w, need_b = ctx.needs_input_grad[:3]
         n, k = wq.shape
-        dx = None
-        if need_x:
-            grad_c = grad.contiguous()
-            if torch.is_grad_enabled() or not _plain(grad_c):  # a graph of the gradient is wanted
+        dx = dw = db = None
+        grad_c = grad.contiguous()
+        if torch.is_grad_enabled() or not _plain(grad_c, x):  # a graph of the gradient is wanted
+            if need_x:
                 dx = grad @ wq
-            else:
-                dx = _matmul(grad_c, ops.transpose_packed(packed, n, k), k, scale, None)
-        dw = grad.t() @ x if need_w else None
-        db = None
+            if need_w:
+                dw = grad.t() @ x
+            if need_b:
+                db = grad.sum(0)
+            return dx, dw, db, None, None
+        if need_x:
+            dx = _matmul(grad_c, ops.transpose_packed(packed, n, k), k, scale, None)
+        if need_w:
+            dw = weight_product(grad_c, x)
         if need_b:
-            db = grad.sum(0) if torch.is_grad_enabled() or not _plain(grad) else ops.column_sum(grad)
+            db = ops.column_sum(grad_c)
         return dx, dw, db, None, None
 
 

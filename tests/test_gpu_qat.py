@@ -116,6 +116,7 @@ STEPS = [(65, 40, 24), (70, 97, 513), (100, 1001, 300), (257, 4096, 512), (96, 6
 @pytest.mark.parametrize("M,K,N", STEPS)
 def test_training_step(gpu, monkeypatch, M, K, N, bias):
     monkeypatch.setattr(qat, "MIN_PRODUCT", 0)
+    monkeypatch.setattr(qat, "MIN_WEIGHTS", 0 if K % 2 == 0 else 1 << 40)
     announce(f"qat step M={M} K={K} N={N} bias={bias}")
     torch.manual_seed(M + K + N)
     layer = layers(N, K, bias, gpu)
@@ -139,7 +140,7 @@ def test_training_step(gpu, monkeypatch, M, K, N, bias):
     close(x.grad, g2 @ wq, N, g2.abs() @ wq.abs(), "dx")
     u = layer.weight.detach() / s
     close(layer.weight.grad, torch.where(u.abs() < 0.5, 2.0 * (g2.T @ x2), torch.zeros_like(wq)),
-          M + 4, 2.0 * (g2.abs().T @ x2.abs()), "dw")
+          6 * M + 4, 2.0 * (g2.abs().T @ x2.abs()), "dw")
     if bias:
         close(layer.bias.grad, g2.sum(0), M, g2.abs().sum(0), "db")
 
@@ -193,3 +194,38 @@ def test_training_routes(gpu, monkeypatch):
     a = layer(x)
     torch.manual_seed(1)
     assert torch.equal(a, F.linear(x, layer._quantize_training_weight(), layer.bias))
+
+
+# M, N, K: one row, a row past a step of 16, columns past a block of 32 and a tile of 256, K that
+# takes no 16-byte stores, the tokens split (few tiles), odd and even step counts
+PRODUCTS = [(1, 1, 1), (17, 33, 40), (32, 256, 32), (100, 257, 300), (1000, 511, 1025),
+            (260, 1030, 258), (1040, 130, 64)]
+
+
+@pytest.mark.parametrize("M,N,K", PRODUCTS)
+def test_weight_product(gpu, monkeypatch, M, N, K):
+    """Six plane products of M exact terms each, summed in float32: within 2 (6 M + 4) 2^-24
+    sum |g x| (doubled for the matrix cores' rounding); the planes left out are below 2^-26
+    of each term, inside the + 4.  Infinities and NaN as the float32 product gives them."""
+    announce(f"qat weight product M={M} N={N} K={K}")
+    monkeypatch.setattr(qat, "MIN_WEIGHTS", 0)
+    gen = torch.Generator("cpu").manual_seed(M + N + K)
+    g = torch.randn((M, N), generator=gen).to(gpu)
+    x = (torch.randn((M, K), generator=gen) * 10.0 ** torch.randint(-3, 4, (M, 1), generator=gen)).to(gpu)
+    want, mags = g.double().T @ x.double(), g.double().abs().T @ x.double().abs()
+    err = (qat.weight_product(g, x).double() - want).abs()
+    assert bool((err <= 2.0 * (6 * M + 4) * U32 * mags + 1e-30).all())
+    ints = torch.randint(-100, 101, (M, N), generator=gen).float().to(gpu)
+    xi = torch.randint(-100, 101, (M, K), generator=gen).float().to(gpu)  # exact sums
+    assert torch.equal(qat.weight_product(ints, xi).double(), ints.double().T @ xi.double())
+    g[M // 2, N // 3] = float("inf")
+    x[M - 1, K // 2] = float("-inf")
+    x[0, 0] = float("nan")
+    got = qat.weight_product(g, x)
+    # of an infinity's products with finite values, all but those with zeros are infinities
+    ref = g.double().T @ x.double()
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+    ok = ref.isfinite()
+    assert bool(((got.double() - ref).abs()[ok] <= 2.0 * (6 * M + 4) * U32 * mags[ok] + 1e-30).all())
+    top = torch.full((M, K), 3.4e38, device=gpu)  # finite, past bf16's largest value
+    assert bool(qat.weight_product(torch.full((M, N), 1e-3 / M, device=gpu), top).isfinite().all())
