@@ -88,9 +88,9 @@ __device__ __forceinline__ float wave_max_dpp(float v) {
 // at once.  Their payload bytes are contiguous and go out as dwords through
 // LDS.  kVec: rows are 16-byte aligned runs of whole float4s, else element loads; columns past
 // the row are zeros.  The slots are private to the wavefront, whose LDS operations complete
-// in order, so no barrier is needed.  8192 x 3072: TQ1_0 28.3 -> 23.1 us, TQ2_0 25.3 ->
-// 20.5 against one block per wavefront with byte gathers; 8192 x 3008 (partial blocks) 62.7
-// -> 21.4, 8191 x 3071 64.3 -> 28.8 against strided loads read twice.
+// in order, so no barrier is needed.  8192 x 3072: TQ1_0 28.2 -> 22.1 us, TQ2_0 25.5 ->
+// 20.7 against one block per wavefront with byte gathers; 8192 x 3008 (partial blocks) 62.7
+// -> 21.3, 8191 x 3071 64.3 -> 28.7 against strided loads read twice.
 template <int Q, bool kVec, int B>
 __global__ __launch_bounds__(256) void tq_quantize_vec_kernel(const float *__restrict__ src,
                                                               uint8_t *__restrict__ dst,

@@ -199,6 +199,43 @@ int main() {
                                                           0, nullptr),
            {T81_HIP_EINVAL_DTYPE});
 
+    // ---- training ----
+    expect("qat scale count", t81_hip_qat_scale(p, 0, kMax, nullptr, f, buf, nullptr),
+           {T81_HIP_EINVAL_SHAPE});
+    expect("qat scale null", t81_hip_qat_scale(p, 0, 4, nullptr, f, nullptr, nullptr),
+           {T81_HIP_EINVAL_POINTER});
+    expect("qat quantize huge", t81_hip_qat_quantize(p, 0, f, 0.5f, p, u8, nullptr, kMax, kMax, nullptr),
+           {T81_HIP_EINVAL_SHAPE});
+    expect("qat quantize thr", t81_hip_qat_quantize(p, 0, f, 2.0f, p, u8, nullptr, 4, 4, nullptr),
+           {T81_HIP_EINVAL_THRESHOLD});
+    expect("qat grad negative", t81_hip_qat_weight_grad(p, 0, f, nullptr, p, kMin, 4, nullptr),
+           {T81_HIP_EINVAL_SHAPE});
+    expect("qat grad dtype", t81_hip_qat_weight_grad(p, T81_DTYPE_I8, f, nullptr, p, 4, 4, nullptr),
+           {T81_HIP_EINVAL_DTYPE});
+    expect("qat matmul huge", t81_hip_qat_matmul(f, u8, f, kMax, kMax, kMax, f, nullptr, p, kMax, nullptr),
+           {T81_HIP_EINVAL_SHAPE});
+    expect("qat matmul ws", t81_hip_qat_matmul(f, u8, f, 4, 4, 4, f, nullptr, nullptr, 0, nullptr),
+           {T81_HIP_EINVAL_POINTER});
+    expect("qat product huge", t81_hip_qat_weight_product(f, f, f, kMax, kMin, kMax, p, kMax, nullptr),
+           {T81_HIP_EINVAL_SHAPE});
+    expect("qat product ws", t81_hip_qat_weight_product(f, f, f, 4, 4, 4, p, 0, nullptr),
+           {T81_HIP_EINVAL_POINTER});
+    expect("column sum huge", t81_hip_column_sum(f, f, kMax, kMax, p, kMax, nullptr),
+           {T81_HIP_EINVAL_SHAPE});
+    expect("column sum scratch", t81_hip_column_sum(f, f, 100, 4, nullptr, 0, nullptr),
+           {T81_HIP_EINVAL_POINTER});
+    for (int64_t v : {kMax, kMin}) {
+        (void)t81_hip_qat_matmul_workspace_size(v, v, v);
+        (void)t81_hip_qat_weight_product_workspace_size(v, v, v);
+        (void)t81_hip_column_sum_scratch_size(v, v);
+        for (int dt : {T81_DTYPE_F32, T81_DTYPE_BF16, T81_DTYPE_I8})
+            for (int64_t m : {int64_t{33}, int64_t{100}, int64_t{2000}}) {
+                (void)t81_hip_ternary_matmul_workspace_size(m, v, 1003, dt);
+                (void)t81_hip_ternary_matmul_workspace_size(m, int64_t{1} << 40, int64_t{1} << 31, dt);
+            }
+    }
+    ++g_cases;
+
     // ---- elementwise ops, transpose, GGUF ----
     expect("where n", t81_hip_where(f, f, f, f, kMin, nullptr), {T81_HIP_EINVAL_SHAPE});
     expect("where null", t81_hip_where(f, nullptr, f, f, 4, nullptr), {T81_HIP_EINVAL_POINTER});
