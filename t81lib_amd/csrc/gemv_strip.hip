@@ -547,6 +547,18 @@ hipError_t launch_strip_x(bool *handled, const void *x, const uint8_t *w, void *
         };
         if (busiest(r - r / 8) < busiest(r)) r -= r / 8;
     }
+    // One token in natural order over three ranges: a CU holds four of its three-wave
+    // workgroups, and a second round of them costs more than longer strips, so past one round
+    // R = 14, then 16, where the launch then is one round.  bf16, K = 4096 at 16384 rows
+    // (1024 workgroups of R = 8) 6.98 us, R = 14 8.06; at 18432 8.92 -> 8.20, 24576 10.25 ->
+    // 9.21, 28672 10.97 -> 9.58, 32768 (R = 16) 12.25 -> 10.47; K = 4500 over 28672 rows
+    // 23.7 -> 15.5.  R = 14 at 32768 rows, 1171 workgroups, 13.23; at 49152 rows, where
+    // neither fits, R stays.
+    if (XT == kDtypeBF16 && m == 1 && S == 8 && nranges == 3 && (r == 7 || r == 8)) {
+        const int64_t held = 4 * static_cast<int64_t>(cu_count());
+        auto blocks = [&](int rr) { return (n + 2 * rr - 1) / (2 * rr); };
+        if (blocks(r) > held) r = blocks(14) <= held ? 14 : (blocks(16) <= held ? 16 : r);
+    }
     if constexpr (XT == kDtypeF32) {
         if (split) {
             // as bf16 at mc = 2 or 4 tokens: padded order, S = 8 / 4, the same hint
