@@ -74,8 +74,12 @@ def ternary(x: torch.Tensor, threshold: float = 0.45, stochastic: bool = False) 
 # ------------------------------------------------------------- the kernels' training step --
 
 def _plain(*tensors: Optional[torch.Tensor]) -> bool:
-    """Ordinary contiguous tensors on the current GPU, outside tracing and forward-mode."""
+    """Ordinary contiguous tensors on the current GPU, outside tracing, dispatch modes (which see
+    tensor operations, not kernels), function transforms and forward-mode."""
     if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return False
+    if torch._C._functorch.peek_interpreter_stack() is not None or \
+            torch._C._len_torch_dispatch_stack() > 0:
         return False
     if torch.autograd.forward_ad._current_level >= 0:
         return False
@@ -88,6 +92,11 @@ def _plain(*tensors: Optional[torch.Tensor]) -> bool:
         if t.device.index != torch.cuda.current_device():
             return False
     return True
+
+
+def _as_saved(t: torch.Tensor, dtype: torch.dtype, *shape: int) -> bool:
+    """Whether a saved tensor came back as it was (saved-tensor hooks may return another)."""
+    return t.dtype == dtype and t.shape == shape and _plain(t)
 
 
 def weight_on_kernels(weight: torch.Tensor, threshold: float) -> bool:
@@ -194,7 +203,10 @@ class TernaryWeight(torch.autograd.Function):
             return None, None, None
         scale, inner = ctx.saved_tensors
         rows, cols = grad.shape
-        if torch.is_grad_enabled() or not _plain(grad):  # a graph of the gradient is wanted
+        if torch.is_grad_enabled() or not _plain(grad) or \
+                not _as_saved(scale, torch.float32) or \
+                not _as_saved(inner, torch.uint16, rows, ops.limbs_for(cols), 4):
+            # a graph of the gradient is wanted, or tensors that the kernel does not take
             shifts = torch.arange(12, device=grad.device, dtype=torch.int32)
             mask = (inner.to(torch.int32).unsqueeze(-1) >> shifts) & 1
             mask = mask.reshape(rows, -1)[:, :cols] != 0
@@ -223,7 +235,11 @@ class TernaryProduct(torch.autograd.Function):
         n, k = wq.shape
         dx = dw = db = None
         grad_c = grad.contiguous()
-        if torch.is_grad_enabled() or not _plain(grad_c, x):  # a graph of the gradient is wanted
+        if torch.is_grad_enabled() or not _plain(grad_c) or \
+                not _as_saved(x, torch.float32, grad.shape[0], k) or \
+                not _as_saved(scale, torch.float32) or \
+                not _as_saved(packed, torch.uint8, n, ops.limbs_for(k), ops.BYTES_PER_LIMB):
+            # a graph of the gradient is wanted, or tensors that the kernels do not take
             if need_x:
                 dx = grad @ wq
             if need_w:

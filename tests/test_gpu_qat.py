@@ -229,3 +229,42 @@ def test_weight_product(gpu, monkeypatch, M, N, K):
     assert bool(((got.double() - ref).abs()[ok] <= 2.0 * (6 * M + 4) * U32 * mags[ok] + 1e-30).all())
     top = torch.full((M, K), 3.4e38, device=gpu)  # finite, past bf16's largest value
     assert bool(qat.weight_product(torch.full((M, N), 1e-3 / M, device=gpu), top).isfinite().all())
+
+
+def test_dispatch_modes(gpu, monkeypatch):
+    """Under a dispatch mode (make_fx) the expression runs, so that its operations are seen."""
+    announce("qat dispatch modes")
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    monkeypatch.setattr(qat, "MIN_PRODUCT", 0)
+    layer = layers(40, 48, True, gpu)
+    x = torch.randn((6, 48), device=gpu)
+    want = F.linear(x, expression(layer.weight, expression_scale(layer.weight, None),
+                                  layer.ternary_threshold), layer.bias)
+    with torch.no_grad():
+        traced = make_fx(lambda v: layer(v))(x)
+        layer.training_scale = None
+        assert torch.allclose(traced(x), want, rtol=1e-5, atol=1e-5)
+    assert any(s in str(n.target) for n in traced.graph.nodes for s in ("mm", "linear"))
+
+
+def test_saved_tensors_of_another_type(gpu, monkeypatch):
+    """Hooks that return another type than was saved: the weight gradient's map by its values, a
+    product of mixed types refused as torch refuses it."""
+    announce("qat saved-tensor hooks")
+    monkeypatch.setattr(qat, "MIN_PRODUCT", 0)
+    layer = layers(40, 48, True, gpu)
+    x = torch.randn((80, 48), device=gpu)
+    with torch.autograd.graph.saved_tensors_hooks(
+            lambda t: t, lambda t: t.to(torch.int32) if t.dtype == torch.uint16 else t):
+        layer(x).sum().backward()
+    got = layer.weight.grad.clone()
+    layer.weight.grad = None
+    layer.training_scale = None
+    layer(x).sum().backward()
+    assert torch.allclose(got, layer.weight.grad, rtol=1e-5, atol=1e-6)
+    with torch.autograd.graph.saved_tensors_hooks(
+            lambda t: t, lambda t: t.bfloat16() if t.shape == x.shape else t):
+        out = layer(x).sum()
+    with pytest.raises(RuntimeError):
+        out.backward()
