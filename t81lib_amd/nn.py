@@ -66,7 +66,9 @@ class Linear(nn.Linear):
     def _training_linear(self, x: torch.Tensor) -> torch.Tensor:
         if self._stochastic_rounding or \
                 type(self)._quantize_training_weight is not Linear._quantize_training_weight or \
-                not qat.weight_on_kernels(self.weight, self.ternary_threshold):
+                type(self)._update_training_scale is not Linear._update_training_scale or \
+                not qat.weight_on_kernels(self.weight, self.ternary_threshold) or \
+                not qat.scale_on_kernels(self.training_scale):
             return F.linear(x, self._quantize_training_weight(), self.bias)
         scale = self._update_training_scale()
         wq, packed = qat.TernaryWeight.apply(self.weight, scale, self.ternary_threshold)

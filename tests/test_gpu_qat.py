@@ -268,3 +268,28 @@ def test_saved_tensors_of_another_type(gpu, monkeypatch):
         out = layer(x).sum()
     with pytest.raises(RuntimeError):
         out.backward()
+
+
+def test_scale_of_other_shapes(gpu, monkeypatch):
+    """A training scale that a program set to more than one value keeps the expression's
+    broadcast (and, for bfloat16 weights, its float32 result): the kernels read one value."""
+    announce("qat scales per row")
+    monkeypatch.setattr(qat, "MIN_PRODUCT", 0)
+    for dtype, shape in [(torch.float32, (40, 1)), (torch.float32, (48,)), (torch.bfloat16, (1,))]:
+        layer = layers(40, 48, False, gpu).to(dtype)
+        x = torch.randn((80, 48), device=gpu)
+        start = torch.rand(shape, device=gpu) * 0.1 + 0.02
+        layer.training_scale = start
+        want = F.linear(x, expression(layer.weight, expression_scale(layer.weight, start),
+                                      layer.ternary_threshold))
+        assert torch.equal(layer(x), want)
+        assert torch.equal(layer.training_scale, expression_scale(layer.weight, start))
+
+    class PerRow(t8nn.Linear):
+        def _update_training_scale(self):
+            return self.weight.detach().abs().amax(1, keepdim=True)
+
+    layer = PerRow(48, 40, bias=False, device=gpu).train()
+    scale = layer._update_training_scale()
+    assert torch.equal(layer(x), F.linear(x, expression(layer.weight, scale,
+                                                        layer.ternary_threshold)))
