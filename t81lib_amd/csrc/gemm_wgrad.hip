@@ -4,10 +4,11 @@
 //
 // on the bf16 matrix cores.  Both operands are split into three bf16 planes that hold them
 // exactly (x = hi + mid + lo, round to nearest), and six of the nine plane products are
-// summed: hi hi, hi mid, mid hi, mid mid, hi lo, lo hi.  The three left out are below 2^-26 of
-// each product.  What bounds it is the matrix pipe: 12 M N K flops at the bf16 rate, against
-// 2 M N K at a float32 rate a tenth of it (2048 x 4096 x 4096: the float32 library product 479-550
-// us, this kernel 298 = 1.38 PFLOP/s, with the images 340; 7.1e-7 from 64 bits against 8.1e-7).
+// summed: hi hi, hi mid, mid hi, mid mid, hi lo, lo hi.  Of the three left out, mid lo and lo mid
+// reach 2^-25 of a product each.  What bounds it is the matrix pipe: 12 M N K flops at the bf16
+// rate, against 2 M N K at a float32 rate a tenth of it (2048 x 4096 x 4096: the float32 library
+// product 479-550 us, this kernel 298 = 1.38 PFLOP/s, with the images 340; 7.1e-7 from 64 bits
+// against 8.1e-7).
 //
 // Plane images, written by a first kernel per operand: pieces of 8 consecutive rows m of one
 // column (16 bytes),
@@ -16,9 +17,11 @@
 // v_mfma_f32_32x32x16_bf16 (32 columns x 16 rows m) is then 1 KB of consecutive bytes, in
 // global memory as in LDS.
 //
-// An infinity times a zero plane of a finite value would be NaN where the float32 product is
-// the infinity, so the image kernels note whether they saw a value that is not finite, and the
-// product then takes such values as zero in every product but hi hi.
+// Plane products overflow where float32 ones need not, with the signs of the residuals, and an
+// infinity times a zero plane is NaN.  So the image kernels note whether they saw a value of
+// 2^53 or more, an infinity or a NaN; below that no sum of fewer than 2^19 products reaches
+// 2^126.  Operands with such a value are multiplied in float32 by a kernel of its own, launched
+// last: of the two products the one that the note does not mean ends at once.
 #include <type_traits>
 
 #include "t81_device.hpp"
@@ -35,6 +38,8 @@ constexpr int kGTile = 256;          // columns of X and of G per workgroup
 constexpr int kGFrags = 48;          // 1 KB fragments per step: 2 x 8 blocks x 3 planes
 constexpr int kGStageStride = 68;
 constexpr uint32_t kGOob = 0x80000000u;
+constexpr uint32_t kGLarge = 0x5A000000u;  // bits of 2^53
+constexpr int64_t kGMostM8 = 65535;        // rows / 8 (M < 2^19)
 
 __global__ void wgrad_clear_kernel(uint32_t *flag) { *flag = 0u; }
 
@@ -54,22 +59,16 @@ __global__ __launch_bounds__(256) void wgrad_image_kernel(const float *__restric
         v[i] = m < M && c < C ? x[static_cast<int64_t>(m) * C + c] : 0.0f;
     }
     bf16x8 pl[3];
-    bool odd = false;
+    bool large = false;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        // |x| past bf16's largest value rounds to it, an infinity or NaN is hi alone
-        const uint32_t u = __float_as_uint(v[i]);
-        const uint32_t mag = u & 0x7FFFFFFFu;
-        uint32_t hb = mag >= 0x7F800000u ? u >> 16 : (u >> 16 & 0x8000u) | 0x7F7Fu;
-        if (mag > 0x7F800000u) hb |= 0x40u;
-        const uint16_t h16 = static_cast<uint16_t>(hb);
-        odd |= mag >= 0x7F800000u;
-        pl[0][i] = mag >= 0x7F7F8000u ? __builtin_bit_cast(__bf16, h16) : static_cast<__bf16>(v[i]);
-        const float r = mag >= 0x7F800000u ? 0.0f : v[i] - static_cast<float>(pl[0][i]);
+        large |= (__float_as_uint(v[i]) & 0x7FFFFFFFu) >= kGLarge;
+        pl[0][i] = static_cast<__bf16>(v[i]);
+        const float r = v[i] - static_cast<float>(pl[0][i]);
         pl[1][i] = static_cast<__bf16>(r);
         pl[2][i] = static_cast<__bf16>(r - static_cast<float>(pl[1][i]));
     }
-    if (odd) *flag = 1u;  // (every writer writes the same)
+    if (large) *flag = 1u;  // (every writer writes the same)
     uint8_t *dst = out + (static_cast<int64_t>(c >> 5) * 3 * M8 + m8) * 512 + (c & 31) * 16;
 #pragma unroll
     for (int p = 0; p < 3; ++p)
@@ -94,18 +93,6 @@ __device__ __forceinline__ void wgrad_load_lds16(const __amdgpu_buffer_rsrc_t sr
         src, (__attribute__((address_space(3))) void *)(dst), 16, offset, 0, 0, 0);
 }
 
-// Eight bf16 with those that are not finite (exponent all ones) as zeros.
-__device__ __forceinline__ u32x4 finite_only(u32x4 v) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t w = v[i];
-        const uint32_t lo = (w & 0x7F80u) == 0x7F80u ? 0u : w & 0xFFFFu;
-        const uint32_t hi = (w & 0x7F800000u) == 0x7F800000u ? 0u : w & 0xFFFF0000u;
-        v[i] = lo | hi;
-    }
-    return v;
-}
-
 // Four waves, one per SIMD, compute 256 columns k of X x 256 columns n of G: wave (wr, wc) owns
 // 128 x 128, 4 x 4 blocks (A = X, B = G, so that a lane's four accumulators are consecutive k
 // of one row n of C).  A step is 16 rows m: 48 KB of fragments, straight copies into one of two
@@ -113,9 +100,6 @@ __device__ __forceinline__ u32x4 finite_only(u32x4 v) {
 // A fragments are read once per step, B fragments once per column block, ahead of their use;
 // the barrier follows chunk 17, past which nothing reads this step's buffer: the last six
 // chunks load the step after next into it and read the next step's first fragments.
-// kCareful: the instance for operands with values that are not finite; the two are launched one
-// after the other and the one that the flag does not mean ends at once.
-template <bool kCareful>
 __global__ __launch_bounds__(256) void gemm_wgrad_kernel(
     const uint8_t *__restrict__ xa, int64_t xa_bytes, const uint8_t *__restrict__ gb,
     int64_t gb_bytes, const uint32_t *__restrict__ flag, float *__restrict__ c, int N, int K,
@@ -124,7 +108,7 @@ __global__ __launch_bounds__(256) void gemm_wgrad_kernel(
     __shared__ __attribute__((aligned(1024))) uint8_t xs1[kGFrags * 1024];
     static_assert(4 * 32 * kGStageStride * 4 <= kGFrags * 1024, "the staging fits a tile buffer");
     static_assert(2 * kGFrags * 1024 + 2048 <= kLdsDmaLimit, "LDS-load targets past 128 KiB");
-    if ((*flag != 0u) != kCareful) return;
+    if (*flag != 0u) return;
     using B0 = std::integral_constant<int, 0>;
     using B1 = std::integral_constant<int, 1>;
     auto tile = [&](auto bufc) -> uint8_t * {
@@ -230,24 +214,17 @@ __global__ __launch_bounds__(256) void gemm_wgrad_kernel(
                         load_part(s + 2, bufc, 2 * (g - 18) + 1);
                     }
                 }
-                u32x4 braw = bq[cb % 2][pb];
-                if (kCareful && pr != 0) braw = finite_only(braw);
-                const bf16x8 bb = __builtin_bit_cast(bf16x8, braw);
+                const bf16x8 bb = __builtin_bit_cast(bf16x8, bq[cb % 2][pb]);
 #pragma unroll
-                for (int rb = 0; rb < 4; ++rb) {
-                    u32x4 araw = a[3 * rb + pa];
-                    if (kCareful && pr != 0) araw = finite_only(araw);
+                for (int rb = 0; rb < 4; ++rb)
                     acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                        __builtin_bit_cast(bf16x8, araw), bb, acc[rb][cb], 0, 0, 0);
-                }
-                if constexpr (!kCareful) {
+                        __builtin_bit_cast(bf16x8, a[3 * rb + pa]), bb, acc[rb][cb], 0, 0, 0);
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
-                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
-                        __builtin_amdgcn_sched_group_barrier(0x006, 2, 0);   // VALU, SALU
-                        __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);   // buffer load
-                    }
+                for (int k = 0; k < 4; ++k) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
+                    __builtin_amdgcn_sched_group_barrier(0x006, 2, 0);   // VALU, SALU
+                    __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);   // buffer load
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 if (g == 17) {
@@ -302,6 +279,112 @@ __global__ __launch_bounds__(256) void gemm_wgrad_kernel(
     }
 }
 
+// The same sums in float32, straight from the operands: 128 x 128 tiles, a wave 64 columns k of
+// X x 64 columns n of G as 2 x 2 blocks of v_mfma_f32_32x32x2_f32 (whose sums run as chains of
+// fused multiply-adds, so that finite terms leave an infinity as it is), 16 rows m a step,
+// double-buffered through registers.  Rows of LDS are 160 floats apart: the two halves of a
+// wave read different banks.  Only for operands of large values: the float32 rate is a tenth
+// of the bf16 one's (2048 x 4096 x 4096 728 us in all, 1623 x 3520 x 1015 214).
+constexpr int kFTile = 128;
+constexpr int kFStep = 16;
+constexpr int kFStride = 160;
+
+__global__ __launch_bounds__(256) void gemm_wgrad_f32_kernel(const float *__restrict__ x,
+                                                             const float *__restrict__ g,
+                                                             const uint32_t *__restrict__ flag,
+                                                             float *__restrict__ c, int M, int N,
+                                                             int K) {
+    __shared__ float xs[2][kFStep][kFStride];
+    __shared__ float gs[2][kFStep][kFStride];
+    if (*flag == 0u) return;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int wr = wave & 1, wc = wave >> 1;
+    const int r = lane & 31;
+    const int h = lane >> 5;
+    const int col = tid & 127;  // of the tile, the column that this thread loads
+    const int row = tid >> 7;   // ... and its rows row, row + 2, ...
+    const int tiles_k = (K + kFTile - 1) / kFTile;
+    const int total = tiles_k * ((N + kFTile - 1) / kFTile);
+    const int steps = (M + kFStep - 1) / kFStep;
+    for (int item = blockIdx.x; item < total; item += gridDim.x) {
+        const int k0 = (item % tiles_k) * kFTile;
+        const int n0 = (item / tiles_k) * kFTile;
+        float rx[kFStep / 2], rg[kFStep / 2];
+        auto load = [&](int s) {
+#pragma unroll
+            for (int i = 0; i < kFStep / 2; ++i) {
+                const int m = kFStep * s + row + 2 * i;
+                rx[i] = m < M && k0 + col < K ? x[static_cast<int64_t>(m) * K + k0 + col] : 0.0f;
+                rg[i] = m < M && n0 + col < N ? g[static_cast<int64_t>(m) * N + n0 + col] : 0.0f;
+            }
+        };
+        auto store = [&](int buf) {
+#pragma unroll
+            for (int i = 0; i < kFStep / 2; ++i) {
+                xs[buf][row + 2 * i][col] = rx[i];
+                gs[buf][row + 2 * i][col] = rg[i];
+            }
+        };
+        floatx16 acc[2][2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+        // (the barrier that ends a step lets the buffer before it be refilled; the last one
+        // covers the next item's first)
+        load(0);
+        store(0);
+        __syncthreads();
+        for (int s = 0; s < steps; ++s) {
+            const int buf = s & 1;
+            if (s + 1 < steps) load(s + 1);
+#pragma unroll
+            for (int m = 0; m < kFStep; m += 2) {
+                float a[2], b[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    a[i] = xs[buf][m + h][64 * wr + 32 * i + r];
+                    b[i] = gs[buf][m + h][64 * wc + 32 * i + r];
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] =
+                            __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+            }
+            if (s + 1 < steps) store(buf ^ 1);
+            __syncthreads();
+        }
+        const bool vec4 = K % 4 == 0 && (reinterpret_cast<uintptr_t>(c) & 15u) == 0;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int n = n0 + 64 * wc + 32 * j + r;
+            if (n >= N) continue;
+            float *cr = c + static_cast<int64_t>(n) * K;
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int a4 = 0; a4 < 4; ++a4) {
+                    const int k = k0 + 64 * wr + 32 * i + 8 * a4 + 4 * h;
+                    if (vec4 && k + 3 < K) {
+                        *reinterpret_cast<f32x4 *>(cr + k) =
+                            f32x4{acc[i][j][4 * a4], acc[i][j][4 * a4 + 1], acc[i][j][4 * a4 + 2],
+                                  acc[i][j][4 * a4 + 3]};
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < 4; ++u)
+                            if (k + u < K) cr[k + u] = acc[i][j][4 * a4 + u];
+                    }
+                }
+        }
+    }
+}
+
 constexpr int64_t kWgradWsBytes = int64_t{1} << 30;
 
 struct WgradPlan {
@@ -321,7 +404,7 @@ WgradPlan wgrad_plan(int64_t m, int64_t n, int64_t k) {
     const int64_t tiles = ((n + kGTile - 1) / kGTile) * ((k + kGTile - 1) / kGTile);
     const int64_t steps = p.m8 / 2;
     // (a grid's second dimension and 32-bit buffer offsets)
-    if (p.m8 > 65535 || p.x_bytes >= 0x40000000 || p.g_bytes >= 0x40000000 || tiles > (int64_t{1} << 24)) return p;
+    if (p.m8 > kGMostM8 || p.x_bytes >= 0x40000000 || p.g_bytes >= 0x40000000 || tiles > (int64_t{1} << 24)) return p;
     int64_t ns = cu_count() / tiles;
     if (ns > steps / 8) ns = steps / 8;
     if (ns < 1) ns = 1;
@@ -362,16 +445,20 @@ hipError_t launch_gemm_wgrad(const float *g, const float *x, float *c, int64_t m
         ((n + kGTile - 1) / kGTile) * ((k + kGTile - 1) / kGTile) * p.nsplit;
     const int64_t cus = cu_count();
     const dim3 grid(static_cast<unsigned>(items < cus ? items : cus));
-    for (auto kernel : {gemm_wgrad_kernel<false>, gemm_wgrad_kernel<true>}) {
-        kernel<<<grid, dim3(256), 0, s>>>(xa, p.x_bytes, gb, p.g_bytes, flag, c,
-                                          static_cast<int>(n), static_cast<int>(k),
-                                          static_cast<int>(p.m8), static_cast<int>(p.sps),
-                                          static_cast<int>(p.nsplit), part);
-        e = hipGetLastError();
+    gemm_wgrad_kernel<<<grid, dim3(256), 0, s>>>(
+        xa, p.x_bytes, gb, p.g_bytes, flag, c, static_cast<int>(n), static_cast<int>(k),
+        static_cast<int>(p.m8), static_cast<int>(p.sps), static_cast<int>(p.nsplit), part);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if (p.nsplit > 1) {
+        e = launch_planes_sum(part, c, n, k, static_cast<int>(p.nsplit), s);
         if (e != hipSuccess) return e;
     }
-    if (p.nsplit == 1) return hipSuccess;
-    return launch_planes_sum(part, c, n, k, static_cast<int>(p.nsplit), s);
+    // (past a split's sum, which then has added nothing that counts)
+    const int64_t f32_tiles = ((n + kFTile - 1) / kFTile) * ((k + kFTile - 1) / kFTile);
+    gemm_wgrad_f32_kernel<<<dim3(static_cast<unsigned>(f32_tiles < 2 * cus ? f32_tiles : 2 * cus)),
+                            dim3(256), 0, s>>>(x, g, flag, c, static_cast<int>(m),
+                                               static_cast<int>(n), static_cast<int>(k));
+    return hipGetLastError();
 }
 
 }  // namespace t81hip
