@@ -30,6 +30,20 @@ constexpr int kPRows = 512;          // weight rows per tile: four waves of 128
 constexpr uint32_t kPOob = 0x80000000u;
 constexpr int kPStageStride = 68;    // floats per staged output row: 64 columns + 4 pad
 
+// Training's product applies a scale to each output that the tensor expression applies to the
+// weights; with trits of one its sums would be 1 / scale larger and overflow where the
+// expression's do not.  Its trits are therefore a power of two (2^-32 .. 1) that keeps every sum
+// within half the expression's size (the other half: hi planes round up), and the rest of the
+// scale (2..4, or a scale of 2 and more as it is) remains for the output.
+__device__ __forceinline__ float scale_of_trits(const float *scale) {
+    if (scale == nullptr) return 1.0f;
+    const int e = static_cast<int>(__float_as_uint(*scale) >> 23 & 0xFFu) - 128;
+    return __uint_as_float(static_cast<uint32_t>(127 + (e < -32 ? -32 : (e < 0 ? e : 0))) << 23);
+}
+__device__ __forceinline__ float scale_of_output(const float *scale) {
+    return scale == nullptr ? 1.0f : *scale / scale_of_trits(scale);
+}
+
 // ---- the plane image ----
 // A wave takes 8 tokens x 8 consecutive pieces: it reads 256 contiguous bytes of each token
 // row (K values of ldx) and writes 128 contiguous bytes per piece and plane.
@@ -162,8 +176,9 @@ __global__ __launch_bounds__(256) void gemm_planes_kernel(
     const int grid = static_cast<int>(gridDim.x);
     const int b = static_cast<int>(blockIdx.x);
     const int pos = grid % 8 == 0 ? (b & 7) * (grid >> 3) + (b >> 3) : b;
-    if (scale != nullptr) alpha *= *scale;
-    lut_fill(lut, tid, 256);  // published by the first item's barrier
+    alpha *= scale_of_output(scale);
+    // (published by the first item's barrier)
+    lut_fill(lut, tid, 256, __float_as_uint(scale_of_trits(scale)) >> 16);
 
     for (int q = pos; q < total; q += grid) {
         const int item = __builtin_amdgcn_readfirstlane(q);
@@ -477,7 +492,7 @@ __global__ __launch_bounds__(256) void planes_sum_kernel(const float *__restrict
                                                          float beta,
                                                          const float *__restrict__ bias,
                                                          const float *__restrict__ scale) {
-    if (scale != nullptr) alpha *= *scale;
+    alpha *= scale_of_output(scale);
     constexpr int V = kVec ? 4 : 1;
     const int64_t total = M * N;
     for (int64_t g = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * V; g < total;

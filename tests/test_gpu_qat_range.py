@@ -1,8 +1,8 @@
 """The training products where float32 overflows: as a float32 product gives them.
 
 The products run as sums over bf16 planes, which must not overflow where the float32 sum does
-not (a hi plane rounds up), and must come out as the infinity, never as infinity - infinity,
-where it does.
+not (a hi plane rounds up, and a training scale below one is applied after the sum), and must
+come out as the infinity, never as infinity - infinity, where it does.
 """
 
 from __future__ import annotations
@@ -12,7 +12,7 @@ import torch
 
 from t81lib_amd import qat
 from test_gpu_exact_f32 import announce
-from test_gpu_qat import PRODUCTS, U32
+from test_gpu_qat import PRODUCTS, U32, expression, expression_scale, layers
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +53,40 @@ def test_weight_product_overflow(gpu, monkeypatch, M, N, K):
     want = 2.0 ** 128 * (1 - 2.0 ** -9) ** 2
     got = qat.weight_product(g, x).double()
     assert bool(((got - want).abs() <= 12 * U32 * want).all())
+
+
+@pytest.mark.parametrize("std", [0.02, 30.0])
+@pytest.mark.parametrize("M,K,N", [(70, 97, 513), (100, 1001, 300), (96, 6000, 130)])
+def test_training_product_overflow(gpu, monkeypatch, M, K, N, std):
+    """Activations and gradients near the largest float32: sums that the scaled weights keep in
+    range stay finite (each output within the float32 summation bound), others do not become
+    NaN."""
+    announce(f"qat product overflow M={M} K={K} N={N} std={std}")
+    monkeypatch.setattr(qat, "MIN_PRODUCT", 0)
+    monkeypatch.setattr(qat, "MIN_WEIGHTS", 1 << 40)
+    torch.manual_seed(M + K + N)
+    layer = layers(N, K, False, gpu)
+    with torch.no_grad():
+        layer.weight.mul_(std / 0.02)
+    top = 3.0e38 / max(1.0, float(layer.weight.detach().abs().max()))
+
+    # ordinary values, and in half the rows about eight near the top
+    def values(rows, cols, scale):
+        v = torch.randn((rows, cols), device=gpu)
+        big = (torch.rand((rows, 1), device=gpu) < 0.5) & (torch.rand((rows, cols), device=gpu) < 8 / cols)
+        return torch.where(big, (0.9 + 0.1 * torch.rand_like(v)) * scale, v)
+
+    x = values(M, K, top).requires_grad_(True)
+    y = layer(x)
+    g = values(M, N, top)
+    y.backward(g)
+    s = expression_scale(layer.weight, None)
+    wq = expression(layer.weight.detach(), s, 0.45).double()
+    for got, a, b in ((y, x.detach(), wq.T), (x.grad, g, wq)):
+        want, mags = a.double() @ b, a.double().abs() @ b.abs()
+        got = got.detach().double()
+        sure = mags < 3.4e38  # no order of the sum overflows
+        assert bool(sure.any()) and not bool(got[sure].isinf().any())
+        assert not bool(got.isnan().any())
+        bound = 2.0 * (a.shape[1] + 2) * U32 * mags + 1e-30
+        assert bool(((got - want).abs() <= bound)[sure].all())
