@@ -747,13 +747,13 @@ hipError_t launch_gemm_exact(const float *x, const uint8_t *w, float *c, int64_t
 }
 
 hipError_t launch_planes_sum(const float *part, float *c, int64_t rows, int64_t cols, int nsplit,
-                             hipStream_t s) {
+                             float alpha, hipStream_t s) {
     const bool v4 = cols % 4 == 0 && reinterpret_cast<uintptr_t>(c) % 16 == 0 &&
                     reinterpret_cast<uintptr_t>(part) % 16 == 0;
     const int64_t threads = rows * cols / (v4 ? 4 : 1);
     const int64_t blocks = (threads + 255) / 256 < 8192 ? (threads + 255) / 256 : 8192;
     auto sum = v4 ? planes_sum_kernel<true> : planes_sum_kernel<false>;
-    sum<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s>>>(part, c, rows, cols, nsplit, 1.0f,
+    sum<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s>>>(part, c, rows, cols, nsplit, alpha,
                                                                   0.0f, nullptr, nullptr);
     return hipGetLastError();
 }

@@ -17,9 +17,12 @@
 // v_mfma_f32_32x32x16_bf16 (32 columns x 16 rows m) is then 1 KB of consecutive bytes, in
 // global memory as in LDS.
 //
+// The operands are multiplied by 2^16 first (and the sums by 2^-32 last): float32 values are
+// multiples of 2^-149 and bf16 ones of 2^-133, so the planes then hold the smallest exactly too.
+//
 // Plane products overflow where float32 ones need not, with the signs of the residuals, and an
 // infinity times a zero plane is NaN.  So the image kernels note whether they saw a value of
-// 2^53 or more, an infinity or a NaN; below that no sum of fewer than 2^19 products reaches
+// 2^37 or more, an infinity or a NaN; below that no sum of fewer than 2^19 products reaches
 // 2^126.  Operands with such a value are multiplied in float32 by a kernel of its own, launched
 // last: of the two products the one that the note does not mean ends at once.
 #include <type_traits>
@@ -38,7 +41,9 @@ constexpr int kGTile = 256;          // columns of X and of G per workgroup
 constexpr int kGFrags = 48;          // 1 KB fragments per step: 2 x 8 blocks x 3 planes
 constexpr int kGStageStride = 68;
 constexpr uint32_t kGOob = 0x80000000u;
-constexpr uint32_t kGLarge = 0x5A000000u;  // bits of 2^53
+constexpr float kGScale = 65536.0f;
+constexpr float kGUnscale = 1.0f / (kGScale * kGScale);
+constexpr uint32_t kGLarge = 0x52000000u;  // bits of 2^37
 constexpr int64_t kGMostM8 = 65535;        // rows / 8 (M < 2^19)
 
 __global__ void wgrad_clear_kernel(uint32_t *flag) { *flag = 0u; }
@@ -63,8 +68,9 @@ __global__ __launch_bounds__(256) void wgrad_image_kernel(const float *__restric
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         large |= (__float_as_uint(v[i]) & 0x7FFFFFFFu) >= kGLarge;
-        pl[0][i] = static_cast<__bf16>(v[i]);
-        const float r = v[i] - static_cast<float>(pl[0][i]);
+        const float y = v[i] * kGScale;
+        pl[0][i] = static_cast<__bf16>(y);
+        const float r = y - static_cast<float>(pl[0][i]);
         pl[1][i] = static_cast<__bf16>(r);
         pl[2][i] = static_cast<__bf16>(r - static_cast<float>(pl[1][i]));
     }
@@ -242,6 +248,7 @@ __global__ __launch_bounds__(256) void gemm_wgrad_kernel(
         // (the last steps' reads of the other buffer fetch unused bytes; no load is pending)
         __syncthreads();  // the staging below overwrites a tile that other waves read from
 
+        const float al = nsplit > 1 ? 1.0f : kGUnscale;
         float *dst = nsplit > 1 ? part + static_cast<int64_t>(sp) * N * K : c;
         const bool vec4 = K % 4 == 0 && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0;
         float *st = reinterpret_cast<float *>(xs0) + wave * (32 * kGStageStride);
@@ -262,7 +269,8 @@ __global__ __launch_bounds__(256) void gemm_wgrad_kernel(
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int row = 4 * i + tq;
-                const f32x4 v = *reinterpret_cast<const f32x4 *>(&st[row * kGStageStride + tc]);
+                const f32x4 t = *reinterpret_cast<const f32x4 *>(&st[row * kGStageStride + tc]);
+                const f32x4 v = {al * t[0], al * t[1], al * t[2], al * t[3]};
                 const int n = n0 + 128 * wc + 32 * cb + row;
                 if (n >= N) continue;
                 float *cr = dst + static_cast<int64_t>(n) * K;
@@ -450,7 +458,7 @@ hipError_t launch_gemm_wgrad(const float *g, const float *x, float *c, int64_t m
         static_cast<int>(p.m8), static_cast<int>(p.sps), static_cast<int>(p.nsplit), part);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (p.nsplit > 1) {
-        e = launch_planes_sum(part, c, n, k, static_cast<int>(p.nsplit), s);
+        e = launch_planes_sum(part, c, n, k, static_cast<int>(p.nsplit), kGUnscale, s);
         if (e != hipSuccess) return e;
     }
     // (past a split's sum, which then has added nothing that counts)

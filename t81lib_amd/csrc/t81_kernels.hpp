@@ -127,9 +127,9 @@ hipError_t launch_gemm_exact(const float *x, const uint8_t *w, float *c, int64_t
                              int64_t k, const float *scale, const float *bias, hipStream_t s,
                              void *ws);
 
-// The row-major rows x cols partials part + sp rows cols, added in split order into c.
+// c = alpha * the sum of the row-major rows x cols partials part + sp rows cols, in split order.
 hipError_t launch_planes_sum(const float *part, float *c, int64_t rows, int64_t cols, int nsplit,
-                             hipStream_t s);
+                             float alpha, hipStream_t s);
 
 // gemm_wgrad.hip: C (n x k) = G^T X for G (m x n), X (m x k), float32; workspace bytes (0: the
 // shape is not taken).

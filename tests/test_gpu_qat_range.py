@@ -55,6 +55,22 @@ def test_weight_product_overflow(gpu, monkeypatch, M, N, K):
     assert bool(((got - want).abs() <= 12 * U32 * want).all())
 
 
+@pytest.mark.parametrize("M,N,K", PRODUCTS)
+def test_weight_product_small_values(gpu, monkeypatch, M, N, K):
+    """Every float32 value is held to its last bit, subnormal ones too: one term per output, so
+    the product is exact."""
+    announce(f"qat weight product small values M={M} N={N} K={K}")
+    monkeypatch.setattr(qat, "MIN_WEIGHTS", 0)
+    gen = torch.Generator("cpu").manual_seed(M + N * 3 + K)
+    exps = torch.randint(-149, -90, (M, K), generator=gen).double()
+    x = (torch.randint(1, 1 << 24, (M, K), generator=gen).double() * 2.0 ** exps).float().to(gpu)
+    one = torch.zeros((M, N))
+    one[torch.randint(0, M, (N,), generator=gen), torch.arange(N)] = 1.0
+    for g, v in ((one.to(gpu), x), (x, one.to(gpu))):
+        got, want = qat.weight_product(g, v), g.double().T @ v.double()
+        assert torch.equal(got.double(), want)
+
+
 @pytest.mark.parametrize("std", [0.02, 30.0])
 @pytest.mark.parametrize("M,K,N", [(70, 97, 513), (100, 1001, 300), (96, 6000, 130)])
 def test_training_product_overflow(gpu, monkeypatch, M, K, N, std):
