@@ -706,7 +706,9 @@ hipError_t launch_planes(const void *x, const uint8_t *w, float *c, int64_t m, i
 // take -- three launches cost 14-18 us whatever the size (1000 -> 1000 at 64 tokens 17.6 ->
 // 18.5, at 65 24.6 -> 18.8; 3072 -> 3072 at 64 20.5 -> 18.6), and at 17..32 tokens the
 // eight-wave kernel's 32-token tiles take 13-26 us (4096 -> 14336 at 32 25.4 -> 26.1, 4096 ->
-// 4096 14.2 -> 18.5).  The size is never less than a token chunk's two planes, 4 bytes a value.
+// 4096 14.2 -> 18.5).  The size is never less than the two planes, 4 bytes a value, of the fewest
+// equal token chunks, within the bound that the plan itself keeps (ceil(m / count) tokens pass
+// it by up to one where that many just fit).
 int64_t gemm_planes_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     if (m <= 32) return 0;
     if (m <= 64 && k % 8 == 0 && (n >= (int64_t{1} << 30) || n * k < (int64_t{1} << 22))) return 0;
@@ -714,7 +716,8 @@ int64_t gemm_planes_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     if (plan.cb == 0) return 0;
     const int64_t per_tok = planes_image_bytes(2, 1, k);
     const int64_t count = (m * per_tok + kPlanesWsBytes - 1) / kPlanesWsBytes;
-    const int64_t chunk = (m + count - 1) / count * per_tok;
+    int64_t chunk = (m + count - 1) / count * per_tok;
+    if (chunk > kPlanesWsBytes) chunk = kPlanesWsBytes;
     return plan.bytes > chunk ? plan.bytes : chunk;
 }
 
