@@ -1341,7 +1341,7 @@ hipError_t launch_gemm_t(const void *x, const uint8_t *w, void *c, int64_t m, in
 //    24 14.5 -> 17.1; 511 -> 700 at 65 15.9 -> 17.0);
 //  * where the split of K over tall tiles does not fit the CUs: few tokens (4096 -> 6144 at
 //    65 / 128 / 256 30.4 -> 23.1 / 30.8 -> 25.2 / 35.6 -> 31.6 us, 14336 -> 4096 at 100
-//    56.6 -> 35.0), items past a round (3072 -> 9216 at 1024, 288 items, 90.2 -> 74.3) or far
+//    56.6 -> 35.0), items past a round (3072 -> 9216 at 600, 270 items, 68.8 -> 51.0) or far
 //    below one (8192 -> 1024 at 512 39.5 -> 30.1).  Where it fits, the split is faster
 //    (14336 -> 4096 at 512 68 -> 86, 4096 -> 6144 at 512 43 -> 52), as it is over fewer than
 //    2 Mi weights (1088 -> 1639 at 96 18.7 -> 20.7) and, past 128 tokens, where C takes no
@@ -1521,12 +1521,14 @@ int64_t gemm_workspace_x(int64_t m, int64_t n, int64_t k) {
         const int64_t eight = gemm_t_workspace<XT, 2, 2, 4, 2>(m, n - n1, k);
         if constexpr (XT == kDtypeI8) return eight > i8 ? eight : i8;
         if constexpr (XT != kDtypeBF16) return eight;
-        // aligned activations whose remaining rows fill a round of half-width tiles run
-        // without a workspace
-        int64_t big = k % 8 == 0 && !gemm_use_half(m, n, n1)
-                          ? split_workspace_bytes(gemm_split_plan(m, n - n1, k))
-                          : 0;
-        if (k % 8 == 0 && n1 == 0) {
+        // aligned activations that tall or 384-row tiles take, or whose remaining rows fill a
+        // round of half-width tiles, run without a workspace
+        int64_t tn1 = 0;
+        bool thalf = false;
+        const bool split = k % 8 == 0 && !gemm_tall_plan(m, n, k, &tn1, &thalf) &&
+                           !gemm_use_384(m, n, k) && !gemm_use_half(m, n, n1);
+        int64_t big = split ? split_workspace_bytes(gemm_split_plan(m, n - n1, k)) : 0;
+        if (split && n1 == 0) {
             // (the tall split's plan, which its tile count can change)
             const int64_t t = split_workspace_bytes(gemm_split_plan_tall(m, n, k));
             if (t > big) big = t;
@@ -1542,10 +1544,8 @@ int64_t gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, int x_dtype) {
     switch (x_dtype) {
         case kDtypeBF16:
             if (gemm_use_plane(m, n, k)) {
-                // (not less than the split's, so a size never shrinks with the path taken)
                 const int64_t plane = gemm_plane_workspace_bytes(m, n, k);
-                const int64_t split = gemm_workspace_x<kDtypeBF16>(m, n, k);
-                if (plane > 0) return plane > split ? plane : split;
+                if (plane > 0) return plane;
             }
             // the column-block stream kernel's shapes (17..gemv_column_blocks_max_tokens
             // tokens, K % 8 == 0): no workspace

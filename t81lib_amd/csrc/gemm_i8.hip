@@ -635,7 +635,11 @@ bool gemm_i8_fits(const void *x, int64_t m, int64_t n, int64_t k) {
            ((m + kI8Tokens - 1) / kI8Tokens) * ((n + kI8Rows - 1) / kI8Rows) < (int64_t(1) << 26);
 }
 
+// (tall and 384-row tiles use none)
 int64_t gemm_i8_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+    int64_t tn1 = 0;
+    bool thalf = false;
+    if ((k <= 8192 && gemm_tall_plan(m, n, k, &tn1, &thalf)) || i8_use_384(m, n, k)) return 0;
     const I8Plan p = i8_plan(m, n, k);
     return p.nsplit > 1 ? p.nsplit * p.tiles * kI8Rows * kI8Tokens * 4 : 0;
 }

@@ -21,3 +21,17 @@ def size(m, n, k, dtype):
 def test_float32_planes_fit_the_scratch(m, k, n):
     """Tokens whose planes are an uneven number of chunks, and K that is cut in parts."""
     assert 0 < size(m, n, k, F32) <= SCRATCH
+
+
+@pytest.mark.parametrize("m,k,n,dtype", [(777, 3072, 9216, BF16), (1024, 3072, 9216, BF16),
+                                         (1024, 4096, 6144, BF16), (1536, 4096, 6144, I8),
+                                         (1024, 3072, 9216, I8), (2500, 14336, 4096, I8)])
+def test_384_row_tiles_use_none(m, k, n, dtype):
+    assert size(m, n, k, dtype) == 0
+
+
+@pytest.mark.parametrize("m,k,n", [(512, 4096, 8448), (65, 2048, 14336), (100, 14336, 4096),
+                                   (2048, 4095, 14336)])
+def test_bf16_images_fit_the_scratch(m, k, n):
+    """The image and its partials, not the split over K that they replace."""
+    assert 0 < size(m, n, k, BF16) <= SCRATCH
