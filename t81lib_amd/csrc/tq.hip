@@ -46,6 +46,15 @@ __device__ __forceinline__ int tq_trit(float v, int use_thr, float thr) {
     return static_cast<int>(r);
 }
 
+// Between a wavefront's LDS writes and its reads of what other lanes wrote.  Its LDS operations
+// complete in order; the fences keep the compiler from moving them (the barrier alone orders
+// no memory).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Row of block b with nb blocks per row (a 64-bit division is a long sequence: 1.7 us of the
 // dequantize's 17 at 8192 x 3072).
 __device__ __forceinline__ int64_t block_row(int64_t b, int64_t nb) {
@@ -87,10 +96,10 @@ __device__ __forceinline__ float wave_max_dpp(float v) {
 // with no carry between its bytes: 13 lanes (TQ1_0) or 16 (TQ2_0) per block, all the blocks
 // at once.  Their payload bytes are contiguous and go out as dwords through
 // LDS.  kVec: rows are 16-byte aligned runs of whole float4s, else element loads; columns past
-// the row are zeros.  The slots are private to the wavefront, whose LDS operations complete
-// in order, so no barrier is needed.  8192 x 3072: TQ1_0 28.2 -> 22.1 us, TQ2_0 25.5 ->
-// 20.7 against one block per wavefront with byte gathers; 8192 x 3008 (partial blocks) 62.7
-// -> 21.3, 8191 x 3071 64.3 -> 28.7 against strided loads read twice.
+// the row are zeros.  The slots are private to the wavefront (wave_lds_sync, no barrier).
+// 8192 x 3072: TQ1_0 28.2 -> 22.1 us, TQ2_0 25.5 -> 20.7 against one block per wavefront with
+// byte gathers; 8192 x 3008 (partial blocks) 62.7 -> 21.3, 8191 x 3071 64.3 -> 28.7 against
+// strided loads read twice.
 template <int Q, bool kVec, int B>
 __global__ __launch_bounds__(256) void tq_quantize_vec_kernel(const float *__restrict__ src,
                                                               uint8_t *__restrict__ dst,
@@ -146,7 +155,7 @@ __global__ __launch_bounds__(256) void tq_quantize_vec_kernel(const float *__res
         slots[wave][64 * u + lane] = dig;
         if (lane == u) out[kHalves * (u + 1) - 1] = __half_as_ushort(__float2half_rn(d));
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
     if (lane < B * kDw) {
         const int u = lane / kDw, o = lane - u * kDw;
         const uint32_t *sd = slots[wave] + 64 * u;
@@ -170,13 +179,13 @@ __global__ __launch_bounds__(256) void tq_quantize_vec_kernel(const float *__res
         out[kHalves * u + 2 * o] = static_cast<uint16_t>(b);
         out[kHalves * u + 2 * o + 1] = static_cast<uint16_t>(b >> 16);
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
     // blk0 is a multiple of B and two blocks are whole dwords: dst + blk0 tq_bytes is 4-byte
     // aligned where dst is
-    const uint32_t *words = reinterpret_cast<const uint32_t *>(out);
     uint32_t *g = reinterpret_cast<uint32_t *>(dst + blk0 * tq_bytes(Q));
     const int halves = n * kHalves;
-    for (int i = lane; i < halves / 2; i += 64) g[i] = words[i];
+    for (int i = lane; i < halves / 2; i += 64)
+        g[i] = out[2 * i] | static_cast<uint32_t>(out[2 * i + 1]) << 16;
     if (halves % 2 != 0 && lane == 0)
         reinterpret_cast<uint16_t *>(g)[halves - 1] = out[halves - 1];
 }
@@ -309,7 +318,7 @@ __global__ __launch_bounds__(256) void tq_dequantize_kernel(const uint8_t *__res
         __shared__ __attribute__((aligned(16))) float turn[4][kQK];
         float *t = turn[threadIdx.x >> 6];
         *reinterpret_cast<floatx4 *>(t + e) = o;
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int64_t col = col0 + 64 * j + lane;
