@@ -17,8 +17,8 @@ weight and its gradient take one pass each instead of about twenty-five, and a f
 product runs over the packed trits with the activations split into three bf16 planes
 that hold them exactly.  Results keep the tensor expression's roundings (weights and
 weight-gradient passes bit for bit); ``weight_on_kernels`` and ``product_on_kernels`` say when
-they stand in, everything else (other devices, subclasses, tracing, forward-mode) runs the
-expression itself.
+they stand in, everything else (other devices, subclasses, tracing, modes, forward-mode) runs
+the expression itself.
 """
 
 from __future__ import annotations
@@ -26,6 +26,7 @@ from __future__ import annotations
 from typing import Optional
 
 import torch
+from torch.utils._device import DeviceContext
 
 from . import _lib, ops
 
@@ -73,15 +74,24 @@ def ternary(x: torch.Tensor, threshold: float = 0.45, stochastic: bool = False) 
 
 # ------------------------------------------------------------- the kernels' training step --
 
-def _plain(*tensors: Optional[torch.Tensor]) -> bool:
-    """Ordinary contiguous tensors on the current GPU, outside tracing, dispatch modes (which see
-    tensor operations, not kernels), function transforms and forward-mode."""
+def observed() -> bool:
+    """Whether something sees or rewrites tensor operations, which kernels would hide from it:
+    tracing, dispatch and torch-function modes, function transforms, forward-mode.  (A device
+    context is a torch-function mode that only fills in the device of new tensors.)"""
     if torch.compiler.is_compiling() or torch.jit.is_tracing():
-        return False
-    if torch._C._functorch.peek_interpreter_stack() is not None or \
-            torch._C._len_torch_dispatch_stack() > 0:
-        return False
-    if torch.autograd.forward_ad._current_level >= 0:
+        return True
+    if torch._C._len_torch_function_stack() > 0 and any(
+            type(m) is not DeviceContext
+            for m in torch.overrides._get_current_function_mode_stack()):
+        return True
+    return (torch._C._len_torch_dispatch_stack() > 0 or
+            torch._C._functorch.peek_interpreter_stack() is not None or
+            torch.autograd.forward_ad._current_level >= 0)
+
+
+def _plain(*tensors: Optional[torch.Tensor]) -> bool:
+    """Ordinary contiguous tensors on the current GPU, and nothing that observes."""
+    if observed():
         return False
     for t in tensors:
         if t is None:

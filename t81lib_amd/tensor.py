@@ -40,6 +40,7 @@ import torch
 from torch import nn
 
 from . import _lib, ops
+from .qat import observed
 
 
 class TritDtype:
@@ -275,13 +276,12 @@ class _TernaryLinearFunction(torch.autograd.Function):
 def _linear_under_grad(ternary: TernaryTensor, x: torch.Tensor,
                        bias: Optional[torch.Tensor]) -> torch.Tensor:
     """x (tokens, cols) @ T^T + bias recorded for autograd."""
-    if (ternary._semantics == "trit_dot" and type(x) in (torch.Tensor, nn.Parameter) and
+    if (not observed() and ternary._semantics == "trit_dot" and type(x) in (torch.Tensor, nn.Parameter) and
             x.is_floating_point() and x.dtype != torch.float64 and x.device.type == "cuda" and
             x.ndim == 2 and x.shape[1] == ternary._k_actual and
             (bias is None or (type(bias) in (torch.Tensor, nn.Parameter) and
                               bias.shape == (ternary._rows,) and bias.device == x.device and
-                              bias.dtype in (torch.float32, torch.bfloat16, torch.float16))) and
-            torch.autograd.forward_ad._current_level < 0):
+                              bias.dtype in (torch.float32, torch.bfloat16, torch.float16)))):
         return _TernaryLinearFunction.apply(ternary, x, bias)
     out = ternary.matmul_input(x)
     return out + bias if bias is not None else out
