@@ -66,29 +66,37 @@ class Linear(nn.Linear):
     def _training_linear(self, x: torch.Tensor) -> torch.Tensor:
         if self._stochastic_rounding or \
                 type(self)._quantize_training_weight is not Linear._quantize_training_weight or \
-                type(self)._update_training_scale is not Linear._update_training_scale or \
-                not qat.weight_on_kernels(self.weight, self.ternary_threshold) or \
-                not qat.scale_on_kernels(self.training_scale):
+                type(self)._update_training_scale is not Linear._update_training_scale:
             return F.linear(x, self._quantize_training_weight(), self.bias)
+        # the weight is read twice, by the scale and here, as the expression reads it: a
+        # parametrized weight may draw random numbers or move its state at each read
         scale = self._update_training_scale()
-        wq, packed = qat.TernaryWeight.apply(self.weight, scale, self.ternary_threshold)
-        if not qat.product_on_kernels(x, self.weight, self.bias):
-            return F.linear(x, wq, self.bias)
-        out = qat.TernaryProduct.apply(x.reshape(-1, x.shape[-1]), wq, self.bias, packed, scale)
+        weight, bias = self.weight, self.bias
+        if not qat.weight_on_kernels(weight, self.ternary_threshold) or \
+                not qat.scale_on_kernels(scale):
+            return F.linear(x, self._ternarized(weight, scale), bias)
+        wq, packed = qat.TernaryWeight.apply(weight, scale, self.ternary_threshold)
+        if not qat.product_on_kernels(x, weight, bias):
+            return F.linear(x, wq, bias)
+        out = qat.TernaryProduct.apply(x.reshape(-1, x.shape[-1]), wq, bias, packed, scale)
         return out.reshape(*x.shape[:-1], out.shape[-1])
 
     def _quantize_training_weight(self) -> torch.Tensor:
         scale = self._update_training_scale()
-        quantized = ternary(self.weight / scale, threshold=self.ternary_threshold,
+        return self._ternarized(self.weight, scale)
+
+    def _ternarized(self, weight: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
+        quantized = ternary(weight / scale, threshold=self.ternary_threshold,
                             stochastic=self._stochastic_rounding)
         return quantized * scale
 
     def _update_training_scale(self) -> torch.Tensor:
-        if qat.weight_on_kernels(self.weight, self.ternary_threshold) and \
+        weight = self.weight
+        if qat.weight_on_kernels(weight, self.ternary_threshold) and \
                 qat.scale_on_kernels(self.training_scale):
-            self.training_scale = qat.training_scale(self.weight, self.training_scale)
+            self.training_scale = qat.training_scale(weight, self.training_scale)
             return self.training_scale
-        candidate = self.weight.detach().abs().amax().clamp(min=1e-6).to(torch.float32)
+        candidate = weight.detach().abs().amax().clamp(min=1e-6).to(torch.float32)
         existing = self.training_scale
         if existing is None or existing.device != candidate.device:
             self.training_scale = candidate
