@@ -64,13 +64,14 @@ class Linear(nn.Linear):
         return self.ternary_weight.linear(x, bias=bias.detach() if bias is not None else None)
 
     def _training_linear(self, x: torch.Tensor) -> torch.Tensor:
+        quantize, update = self._quantize_training_weight, self._update_training_scale
         if self._stochastic_rounding or \
-                type(self)._quantize_training_weight is not Linear._quantize_training_weight or \
-                type(self)._update_training_scale is not Linear._update_training_scale:
-            return F.linear(x, self._quantize_training_weight(), self.bias)
+                getattr(quantize, "__func__", None) is not Linear._quantize_training_weight or \
+                getattr(update, "__func__", None) is not Linear._update_training_scale:
+            return F.linear(x, quantize(), self.bias)
         # the weight is read twice, by the scale and here, as the expression reads it: a
         # parametrized weight may draw random numbers or move its state at each read
-        scale = self._update_training_scale()
+        scale = update()
         weight, bias = self.weight, self.bias
         if not qat.weight_on_kernels(weight, self.ternary_threshold) or \
                 not qat.scale_on_kernels(scale):

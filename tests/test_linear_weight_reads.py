@@ -53,3 +53,12 @@ def test_random_weight_repeats(device):
     q = torch.where(u.abs() >= layer.ternary_threshold, u.sign(), torch.zeros_like(u))
     want = nn.functional.linear(x, q * scale, layer.bias)
     torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_replaced_on_one_layer(device):
+    """A layer whose own quantizer a program replaced uses it."""
+    layer = t8nn.Linear(48, 40, bias=False, device=device).train()
+    layer._quantize_training_weight = lambda: torch.ones((40, 48), device=device)
+    x = torch.randn((5, 48), device=device)
+    assert torch.equal(layer(x), nn.functional.linear(x, torch.ones((40, 48), device=device)))
