@@ -90,14 +90,16 @@ def observed() -> bool:
 
 
 def _plain(*tensors: Optional[torch.Tensor]) -> bool:
-    """Ordinary contiguous tensors on the current GPU, and nothing that observes."""
+    """Ordinary contiguous tensors on the current GPU, and nothing that observes.  (A batch of
+    gradients taken through one graph at once has no storage of its own.)"""
     if observed():
         return False
     for t in tensors:
         if t is None:
             continue
         if type(t) not in (torch.Tensor, torch.nn.Parameter) or t.device.type != "cuda" or \
-                t.layout != torch.strided or not t.is_contiguous():
+                t.layout != torch.strided or not torch._C._has_storage(t) or \
+                not t.is_contiguous():
             return False
         if t.device.index != torch.cuda.current_device():
             return False

@@ -268,8 +268,9 @@ class _TernaryLinearFunction(torch.autograd.Function):
         if ctx.needs_input_grad[1]:
             dx = ops.ternary_matmul(g, t.transposed_packed(), t._rows)
         if ctx.needs_input_grad[2]:
-            # (a graph of the gradient, where one is wanted, comes from the tensor sum)
-            db = g.sum(0) if torch.is_grad_enabled() else ops.column_sum(g)
+            # (a graph of the gradient, or a batch of them, comes from the tensor sum)
+            plain = not torch.is_grad_enabled() and not observed() and torch._C._has_storage(g)
+            db = ops.column_sum(g) if plain else g.sum(0)
         return None, dx, db
 
 
