@@ -370,19 +370,6 @@ constexpr uint32_t kW4Oob = 0x80000000u;
 constexpr int kW4StageStride = 68;   // floats per staged output row: 64 columns + 4 pad
 constexpr int kW4StageBytes = 4 * 32 * kW4StageStride * 4;   // four waves' staging regions
 
-// A raw buffer descriptor over [base, base + bytes) (clamped to 2^31 - 1 bytes) whose
-// fields are forced into scalar registers: the loads then need no per-lane
-// descriptor checks.  base and bytes must be the same in every lane.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const void *base, int64_t bytes) {
-    const uint64_t p = reinterpret_cast<uint64_t>(base);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p));
-    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p >> 32));
-    const int n = __builtin_amdgcn_readfirstlane(bytes < 0x7FFFFFFF ? static_cast<int>(bytes)
-                                                                    : 0x7FFFFFFF);
-    return __builtin_amdgcn_make_buffer_rsrc(
-        reinterpret_cast<void *>((static_cast<uint64_t>(hi) << 32) | lo), 0, n, 0x00020000);
-}
-
 // Work items.  Weight rows [0, n1) run as whole 256 x 256 tiles (512 x 128 for WR = 4;
 // all k-steps, result to C).  Rows [n1, N) run either as split-K items (nsplit > 0): item
 // (split sp, tile t of that region) runs k-steps [sp * sps, (sp + 1) * sps) and stores its

@@ -57,16 +57,6 @@ constexpr int kI8LutBytes = 32 * 256 * 8;
 
 static_assert(kI8Tokens * kI8RowSlots % (64 * 4) == 0, "tile loads must split evenly");
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t i8_rsrc(const void *base, int64_t bytes) {
-    const uint64_t p = reinterpret_cast<uint64_t>(base);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p));
-    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p >> 32));
-    const int n = __builtin_amdgcn_readfirstlane(bytes < 0x7FFFFFFF ? static_cast<int>(bytes)
-                                                                    : 0x7FFFFFFF);
-    return __builtin_amdgcn_make_buffer_rsrc(
-        reinterpret_cast<void *>((static_cast<uint64_t>(hi) << 32) | lo), 0, n, 0x00020000);
-}
-
 // Three int8 trits of tryte u (u = 13 + t0 + 3 t1 + 9 t2) in bytes 0-2, zero past 26.
 __device__ __forceinline__ uint32_t i8_trits(int u) {
     if (u >= 27) return 0u;
@@ -180,7 +170,7 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
 
         // weights: rows past N read zeros; a limb past L (odd L, last step) reads the next
         // row's first limb or zeros -- finite trits that meet zero activations
-        const __amdgpu_buffer_rsrc_t wsrc = i8_rsrc(w + static_cast<int64_t>(nwg) * L * kTrytes,
+        const __amdgpu_buffer_rsrc_t wsrc = uniform_rsrc(w + static_cast<int64_t>(nwg) * L * kTrytes,
                                                     static_cast<int64_t>(N - nwg) * L * kTrytes);
         uint32_t woff[RB];
 #pragma unroll
@@ -197,7 +187,7 @@ __global__ __launch_bounds__(kI8Threads) void gemm_w4_i8_kernel(
 
         // activation tile: load i of wave w fills slots q = 64 (LPW w + i) + lane, tile row
         // q / 7, slot q % 7; tokens past M read zeros (buffer based at token m0)
-        const __amdgpu_buffer_rsrc_t xsrc = i8_rsrc(x + static_cast<int64_t>(m0) * K,
+        const __amdgpu_buffer_rsrc_t xsrc = uniform_rsrc(x + static_cast<int64_t>(m0) * K,
                                                     static_cast<int64_t>(M - m0) * K);
         uint32_t tbase[LPW];
         uint32_t tslot[(LPW + 3) / 4];

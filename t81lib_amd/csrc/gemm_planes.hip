@@ -107,23 +107,6 @@ __global__ __launch_bounds__(256) void planes_kernel(
             __builtin_bit_cast(u32x4, pl[q]);
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const void *base, int64_t bytes) {
-    const uint64_t p = reinterpret_cast<uint64_t>(base);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p));
-    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p >> 32));
-    const int n = __builtin_amdgcn_readfirstlane(bytes < 0x7FFFFFFF ? static_cast<int>(bytes)
-                                                                    : 0x7FFFFFFF);
-    return __builtin_amdgcn_make_buffer_rsrc(
-        reinterpret_cast<void *>((static_cast<uint64_t>(hi) << 32) | lo), 0, n, 0x00020000);
-}
-
-// 16 bytes per lane from the buffer into LDS at dst + 16 lane, through no register.
-__device__ __forceinline__ void load_lds16(const __amdgpu_buffer_rsrc_t src, uint8_t *dst,
-                                           uint32_t offset) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        src, (__attribute__((address_space(3))) void *)(dst), 16, offset, 0, 0, 0);
-}
-
 // ---- the product ----
 // A workgroup of four waves (one per SIMD) computes 512 weight rows x 32 CB tokens of C^T,
 // wave w rows 128 w .. of all the tokens: 4 x CB blocks of v_mfma_f32_32x32x16_bf16.  A half
@@ -202,7 +185,7 @@ __global__ __launch_bounds__(256) void gemm_planes_kernel(
         // (odd L) reads the next row's first limb or zeros, finite trits that meet zero
         // activations.
         const __amdgpu_buffer_rsrc_t wsrc =
-            plane_rsrc(w + static_cast<int64_t>(nwg) * pitch * kTrytes,
+            uniform_rsrc(w + static_cast<int64_t>(nwg) * pitch * kTrytes,
                        (static_cast<int64_t>(N - 1 - nwg) * pitch + L) * kTrytes);
         uint32_t woff[RB];
 #pragma unroll
@@ -220,7 +203,7 @@ __global__ __launch_bounds__(256) void gemm_planes_kernel(
         // Tile load i of a wave: fragment f = 4 i + wave of the tile, token block f / 3P, plane
         // and j from f % 3P: lane (h, r) takes piece 12 t + 3 half + 6 h + j of token r.
         // Blocks and tokens past M, pieces past K and spare loads are out of range.
-        const __amdgpu_buffer_rsrc_t xsrc = plane_rsrc(xp, xp_bytes);
+        const __amdgpu_buffer_rsrc_t xsrc = uniform_rsrc(xp, xp_bytes);
         const uint32_t lane16 = static_cast<uint32_t>(lane) * 16u;
         uint32_t loff[LPW];
         int piece[LPW];  // bytes between pieces

@@ -82,23 +82,6 @@ __global__ __launch_bounds__(256) void wgrad_image_kernel(const float *__restric
             __builtin_bit_cast(u32x4, pl[p]);
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t wgrad_rsrc(const void *base, int64_t bytes) {
-    const uint64_t p = reinterpret_cast<uint64_t>(base);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p));
-    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p >> 32));
-    const int n = __builtin_amdgcn_readfirstlane(bytes < 0x7FFFFFFF ? static_cast<int>(bytes)
-                                                                    : 0x7FFFFFFF);
-    return __builtin_amdgcn_make_buffer_rsrc(
-        reinterpret_cast<void *>((static_cast<uint64_t>(hi) << 32) | lo), 0, n, 0x00020000);
-}
-
-// 16 bytes per lane from the buffer into LDS at dst + 16 lane, through no register.
-__device__ __forceinline__ void wgrad_load_lds16(const __amdgpu_buffer_rsrc_t src, uint8_t *dst,
-                                                 uint32_t offset) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        src, (__attribute__((address_space(3))) void *)(dst), 16, offset, 0, 0, 0);
-}
-
 // Four waves, one per SIMD, compute 256 columns k of X x 256 columns n of G: wave (wr, wc) owns
 // 128 x 128, 4 x 4 blocks (A = X, B = G, so that a lane's four accumulators are consecutive k
 // of one row n of C).  A step is 16 rows m: 48 KB of fragments, straight copies into one of two
@@ -152,8 +135,8 @@ __global__ __launch_bounds__(256) void gemm_wgrad_kernel(
         const int r = lane & 31;
         const int h = lane >> 5;
         const uint32_t lane16 = static_cast<uint32_t>(lane) * 16u;
-        const __amdgpu_buffer_rsrc_t asrc = wgrad_rsrc(xa, xa_bytes);
-        const __amdgpu_buffer_rsrc_t bsrc = wgrad_rsrc(gb, gb_bytes);
+        const __amdgpu_buffer_rsrc_t asrc = uniform_rsrc(xa, xa_bytes);
+        const __amdgpu_buffer_rsrc_t bsrc = uniform_rsrc(gb, gb_bytes);
         // load i of a wave: fragment f = 4 i + wave; f < 24 of X, block f / 3, plane f % 3
         uint32_t fbase[12];
 #pragma unroll
@@ -166,8 +149,8 @@ __global__ __launch_bounds__(256) void gemm_wgrad_kernel(
                                  : kGOob;
         }
         auto load_part = [&](int s, auto bufc, int i) {
-            wgrad_load_lds16(i < 6 ? asrc : bsrc, &tile(bufc)[1024 * (4 * i + wave)],
-                             lane16 + (fbase[i] + static_cast<uint32_t>(s) * 1024u));
+            load_lds16(i < 6 ? asrc : bsrc, &tile(bufc)[1024 * (4 * i + wave)],
+                       lane16 + (fbase[i] + static_cast<uint32_t>(s) * 1024u));
         };
         auto read_a = [&](auto bufc, int f) -> u32x4 {  // f = rb * 3 + plane
             return *reinterpret_cast<const u32x4 *>(&tile(bufc)[(12 * wr + f) * 1024 + lane16]);

@@ -101,6 +101,26 @@ static_assert(waitcnt_vm<4>() == 0x0F74 && waitcnt_vm<9>() == 0x0F79, "gfx9 s_wa
 // object below this bound (their total static LDS <= kLdsDmaLimit, checked where declared).
 constexpr int kLdsDmaLimit = 128 * 1024;
 
+// A raw buffer descriptor over [base, base + bytes) (clamped to 2^31 - 1 bytes) whose
+// fields are forced into scalar registers: the loads then need no per-lane
+// descriptor checks.  base and bytes must be the same in every lane.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const void *base, int64_t bytes) {
+    const uint64_t p = reinterpret_cast<uint64_t>(base);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p >> 32));
+    const int n = __builtin_amdgcn_readfirstlane(bytes < 0x7FFFFFFF ? static_cast<int>(bytes)
+                                                                    : 0x7FFFFFFF);
+    return __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<void *>((static_cast<uint64_t>(hi) << 32) | lo), 0, n, 0x00020000);
+}
+
+// 16 bytes per lane from the buffer into LDS at dst + 16 lane, through no register.
+__device__ __forceinline__ void load_lds16(const __amdgpu_buffer_rsrc_t src, uint8_t *dst,
+                                           uint32_t offset) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        src, (__attribute__((address_space(3))) void *)(dst), 16, offset, 0, 0, 0);
+}
+
 __device__ __forceinline__ uint16_t bf16_bits_rne(float f) {
     // round-to-nearest-even float -> bf16 (NaN kept quiet)
     uint32_t u = __float_as_uint(f);
