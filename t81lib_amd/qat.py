@@ -26,6 +26,7 @@ from __future__ import annotations
 from typing import Optional
 
 import torch
+from torch.nn import functional as F
 from torch.utils._device import DeviceContext
 
 from . import _lib, ops
@@ -157,12 +158,23 @@ def _workspace(m: int, n: int, k: int) -> int:
     return int(_lib.lib().t81_hip_qat_matmul_workspace_size(m, n, k))
 
 
+def _scratch(nbytes: int, device: torch.device) -> Optional[torch.Tensor]:
+    """None where the device has no room for it: the library's product then runs, which needs
+    none (the planes take up to 512 MiB, the weight gradient's 1 GiB)."""
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def _matmul(x: torch.Tensor, packed: torch.Tensor, n: int, scale: torch.Tensor,
-            bias: Optional[torch.Tensor]) -> torch.Tensor:
+            bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     m, k = x.shape
-    out = torch.empty((m, n), dtype=torch.float32, device=x.device)
     need = _workspace(m, n, k)
-    ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+    ws = _scratch(need, x.device)
+    if ws is None:
+        return None
+    out = torch.empty((m, n), dtype=torch.float32, device=x.device)
     _lib.check(_lib.lib().t81_hip_qat_matmul(
         x.data_ptr(), packed.data_ptr(), out.data_ptr(), m, n, k, scale.data_ptr(),
         bias.data_ptr() if bias is not None else None, ws.data_ptr(), need, ops._stream()))
@@ -181,10 +193,10 @@ def weight_product(grad: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     (m, n), k = grad.shape, x.shape[1]
     lib = _lib.lib()
     need = lib.t81_hip_qat_weight_product_workspace_size(m, n, k) if n * k >= MIN_WEIGHTS else 0
-    if need == 0:  # (or operands whose planes pass the workspace's bound)
+    ws = _scratch(need, x.device) if need > 0 else None
+    if ws is None:  # (or operands whose planes pass the workspace's bound)
         return grad.t() @ x
     out = torch.empty((n, k), dtype=torch.float32, device=x.device)
-    ws = torch.empty(need, dtype=torch.uint8, device=x.device)
     _lib.check(lib.t81_hip_qat_weight_product(grad.data_ptr(), x.data_ptr(), out.data_ptr(), m, n,
                                               k, ws.data_ptr(), need, ops._stream()))
     return out
@@ -238,7 +250,8 @@ class TernaryProduct(torch.autograd.Function):
     def forward(ctx, x: torch.Tensor, wq: torch.Tensor, bias: Optional[torch.Tensor],
                 packed: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
         ctx.save_for_backward(x, wq, packed, scale)
-        return _matmul(x, packed, wq.shape[0], scale, bias)
+        out = _matmul(x, packed, wq.shape[0], scale, bias)
+        return F.linear(x, wq, bias) if out is None else out
 
     @staticmethod
     def backward(ctx, grad: torch.Tensor):
@@ -261,6 +274,8 @@ class TernaryProduct(torch.autograd.Function):
             return dx, dw, db, None, None
         if need_x:
             dx = _matmul(grad_c, ops.transpose_packed(packed, n, k), k, scale, None)
+            if dx is None:
+                dx = grad_c @ wq
         if need_w:
             dw = weight_product(grad_c, x)
         if need_b:
