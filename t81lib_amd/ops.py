@@ -225,7 +225,12 @@ def ternary_matmul(x: torch.Tensor, w_packed: torch.Tensor, k: Optional[int] = N
     # Split K and the activations' plane images use a workspace from torch's caching
     # allocator (safe under graph capture); its size is 0 for the other shapes.
     ws_bytes = lib.t81_hip_ternary_matmul_workspace_size(m, n, k, code)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes > 0 else None
+    ws = None
+    if ws_bytes > 0:
+        try:
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+        except torch.OutOfMemoryError:  # every shape runs without one too
+            ws_bytes = 0
     rc = lib.t81_hip_ternary_matmul_ws(which, x.data_ptr(), code, w_packed.data_ptr(),
                                        c.data_ptr(), m, n, k, alpha, beta, bias_ptr,
                                        ws.data_ptr() if ws is not None else None, ws_bytes,

@@ -8,6 +8,7 @@ import torch
 
 from t81lib_amd import qat
 from test_gpu_exact_f32 import announce
+from test_gpu_matmul_memory import no_room_for
 from test_gpu_qat import layers
 
 pytestmark = pytest.mark.gpu
@@ -29,19 +30,12 @@ def test_step_without_room_for_workspaces(gpu, monkeypatch):
         return y.detach(), x.grad, layer.weight.grad, layer.bias.grad
 
     want = step()
-    total = torch.cuda.get_device_properties(gpu).total_memory
     real, asked = qat._scratch, []
 
-    def scratch(nbytes, device):  # with 16 MiB left on the device
-        torch.cuda.empty_cache()
-        torch.cuda.set_per_process_memory_fraction(
-            (torch.cuda.memory_reserved() + (16 << 20)) / total)
-        try:
-            ws = real(nbytes, device)
-        finally:
-            torch.cuda.set_per_process_memory_fraction(1.0)
-        asked.append((nbytes, ws))
-        return ws
+    def scratch(nbytes, device):
+        with no_room_for(16 << 20, device):
+            asked.append((nbytes, real(nbytes, device)))
+        return asked[-1][1]
 
     monkeypatch.setattr(qat, "_scratch", scratch)
     got = step()
