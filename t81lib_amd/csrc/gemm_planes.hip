@@ -40,6 +40,16 @@ __device__ __forceinline__ float scale_of_trits(const float *scale) {
     const int e = static_cast<int>(__float_as_uint(*scale) >> 23 & 0xFFu) - 128;
     return __uint_as_float(static_cast<uint32_t>(127 + (e < -32 ? -32 : (e < 0 ? e : 0))) << 23);
 }
+// Turns the trits of ones that lut_fill wrote into that power of two (each thread the words it
+// wrote itself).
+__device__ __forceinline__ void lut_scale(uint8_t *lds, int tid, int nthreads, float size) {
+    const uint32_t one = __float_as_uint(size) >> 16;
+    uint32_t *words = reinterpret_cast<uint32_t *>(lds);
+    for (int i = tid; i < kLutBytes / 4; i += nthreads) {
+        const uint32_t w = words[i];
+        words[i] = (w & 0x80008000u) | (w & 0x7FFFu ? one : 0u) | (w & 0x7FFF0000u ? one << 16 : 0u);
+    }
+}
 __device__ __forceinline__ float scale_of_output(const float *scale) {
     return scale == nullptr ? 1.0f : *scale / scale_of_trits(scale);
 }
@@ -160,8 +170,8 @@ __global__ __launch_bounds__(256) void gemm_planes_kernel(
     const int b = static_cast<int>(blockIdx.x);
     const int pos = grid % 8 == 0 ? (b & 7) * (grid >> 3) + (b >> 3) : b;
     alpha *= scale_of_output(scale);
-    // (published by the first item's barrier)
-    lut_fill(lut, tid, 256, __float_as_uint(scale_of_trits(scale)) >> 16);
+    lut_fill(lut, tid, 256);  // published by the first item's barrier
+    if (scale != nullptr) lut_scale(lut, tid, 256, scale_of_trits(scale));
 
     for (int q = pos; q < total; q += grid) {
         const int item = __builtin_amdgcn_readfirstlane(q);

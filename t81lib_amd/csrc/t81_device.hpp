@@ -20,8 +20,12 @@ __host__ __device__ constexpr int trit_of(int u, int p) {
     return p == 0 ? (u % 3) - 1 : (p == 1 ? ((u / 3) % 3) - 1 : (u / 9) - 1);
 }
 
+__host__ __device__ constexpr uint32_t bf16_bits_of_trit(int t) {
+    return t > 0 ? 0x3F80u : (t < 0 ? 0xBF80u : 0u);
+}
+
 // ---------------------------------------------------------------------------
-// Decode tables in LDS, trits as bf16.  For a byte u (one tryte = trits t0,t1,t2):
+// Decode tables in LDS.  For a byte u (one tryte = trits t0,t1,t2):
 //   E[u] = { bf16(t0) | bf16(t1) << 16,  bf16(t2) }
 //   F[u] = { bf16(t0) << 16,             bf16(t1) | bf16(t2) << 16 }
 // Two consecutive bytes (a, b) hold trits 0..5 of a 6-trit run; the three
@@ -36,10 +40,8 @@ constexpr int kLutBytes = 256 + 256 + 16;   // F start + max field + one entry
 
 // Writes the E/F tables (and the zero fill around them) with one pass: thread i
 // owns word i, so no barrier is needed between fill and entries.  The caller
-// issues the __syncthreads() that publishes the table.  one: the bf16 bits that a trit of +1
-// decodes to.
-__device__ __forceinline__ void lut_fill(uint8_t *lds, int tid, int nthreads,
-                                         uint32_t one = 0x3F80u) {
+// issues the __syncthreads() that publishes the table.
+__device__ __forceinline__ void lut_fill(uint8_t *lds, int tid, int nthreads) {
     uint32_t *words = reinterpret_cast<uint32_t *>(lds);
     for (int i = tid; i < kLutBytes / 4; i += nthreads) {
         const int off = 4 * i;
@@ -49,10 +51,9 @@ __device__ __forceinline__ void lut_fill(uint8_t *lds, int tid, int nthreads,
         const int u = rel / 8;
         const int part = (rel % 8) / 4;
         if (rel >= 0 && u < 27 && off < kLutF + 8 * 27) {
-            auto bits = [&](int t) { return t > 0 ? one : (t < 0 ? one | 0x8000u : 0u); };
-            const uint32_t b0 = bits(trit_of(u, 0));
-            const uint32_t b1 = bits(trit_of(u, 1));
-            const uint32_t b2 = bits(trit_of(u, 2));
+            const uint32_t b0 = bf16_bits_of_trit(trit_of(u, 0));
+            const uint32_t b1 = bf16_bits_of_trit(trit_of(u, 1));
+            const uint32_t b2 = bf16_bits_of_trit(trit_of(u, 2));
             if (in_e) v = part == 0 ? (b0 | (b1 << 16)) : b2;
             else v = part == 0 ? (b0 << 16) : (b1 | (b2 << 16));
         }
