@@ -356,7 +356,8 @@ int t81_hip_qat_weight_grad(const void *g, int g_dtype, const float *scale,
                             void *stream);
 
 /* c[m, n] = *scale * sum_k x[m, k] * T[n, k] + bias[n], float32, with x split into three bf16
- * planes that hold it exactly (products exact, float32 sums).  workspace (16-byte aligned):
+ * planes that hold it exactly, but for digits below 2^-133 (products exact, float32 sums; no
+ * sum overflows where that of x * (*scale * T) does not).  workspace (16-byte aligned):
  * t81_hip_qat_matmul_workspace_size bytes; 0 there: the shape is not taken (EINVAL_SHAPE).
  * Replaces: the F.linear of t81/nn/linear.py:93-99 and its input gradient (with the
  * transposed limbs). */
@@ -367,7 +368,8 @@ int t81_hip_qat_matmul(const float *x, const uint8_t *w, float *c, int64_t m, in
 
 /* c[n, k] = sum_m g[m, n] * x[m, k] (float32, row-major; the weight's gradient of that
  * product), both operands split into three bf16 planes that hold them exactly and the six
- * largest plane products summed in float32.  workspace (16-byte aligned):
+ * largest plane products summed in float32 (the rest below 2^-24 of a term); with a value of 2^37
+ * or more, an infinity or a NaN among them, in float32 throughout.  workspace (16-byte aligned):
  * t81_hip_qat_weight_product_workspace_size bytes; 0 there: not taken (EINVAL_SHAPE). */
 int64_t t81_hip_qat_weight_product_workspace_size(int64_t m, int64_t n, int64_t k);
 int t81_hip_qat_weight_product(const float *g, const float *x, float *c, int64_t m, int64_t n,

@@ -6,8 +6,9 @@
 // ~N*K/3 weight bytes), so the kernel is built around v_mfma_f32_32x32x16_bf16.
 // Decoded trits (-1, 0, +1) are exact in bf16; bf16 activations feed the MFMA
 // directly, fp32 activations as a hi + lo bf16 pair (two MFMAs, |error| <=
-// 2^-18 |x| per product; past 32 tokens, given a workspace, gemm_planes.hip), int8 activations exactly (fp32 sums of integers stay
-// exact while |sum| < 2^24, which the ABI enforces through K <= 131071).
+// 2^-17 |x| per product; past 32 tokens, given a workspace, gemm_planes.hip), int8 activations
+// exactly (fp32 sums of integers stay exact while |sum| < 2^24, which the ABI enforces through
+// K <= 131071).
 //
 // Tiling.  A workgroup of WN x WM waves computes a (32*RN*WN) x (32*CM*WM)
 // tile of C^T (weight rows x tokens).  Per k-step of LK limbs (48 * LK trits):
@@ -1040,9 +1041,9 @@ int64_t split_workspace_bytes(const SplitPlan &p) {
 //    tile each (qkv at M = 2048: 192 -> 256 tiles, 83.2 -> 80.7 us, with beta = 1 95.4 -> 89.8;
 //    3072 -> 3072 at M = 4096 66.2 -> 64.7).
 //  * of a shape with fewer, up to K = 8192, instead of a split of K and its sum: from 160 of
-//    them (3072 -> 9216 at M = 777 58.7 -> 51.9 us, at 1024 90.1 -> 54.6, 4096 -> 6144 at 1300
-//    104.5 -> 66.0, 2048 -> 8192 at 1024 51.3 -> 43.2), or from half a round where the split's
-//    items run past a round of the CUs (4096 -> 6144 at 1024, 96 tall tiles x 3, 79.8 -> 66.0).
+//    them (3072 -> 9216 at M = 777 62.9 -> 54.6 us, at 1024 91.5 -> 54.5, 4096 -> 6144 at 1300
+//    106.5 -> 64.3, 2048 -> 8192 at 1024 52.4 -> 42.1), or from half a round where the split's
+//    items run past a round of the CUs (4096 -> 6144 at 1024, 96 tall tiles x 3, 80.8 -> 59.4).
 //    Not below (4096 -> 4096 at 1700, 154 of them, 65.5 -> 69.5), nor over K = 14336, whose
 //    partials weigh less beside its steps (2048 tokens 188 -> 239).
 bool gemm_use_384(int64_t m, int64_t n, int64_t k) {
@@ -1323,13 +1324,13 @@ hipError_t launch_gemm_t(const void *x, const uint8_t *w, void *c, int64_t m, in
 // x.  The image costs a pass over x, and its product takes any K and x, in 64-token tiles
 // too.  Taken
 //  * where K is no multiple of 8 (element loads into the eight-wave kernel otherwise): 4095 ->
-//    14336 at 2048 tokens 774 -> 212 us, at 48 47 -> 26; 1003 -> 1001 at 128 26 -> 21; not
+//    14336 at 2048 tokens 765 -> 219 us, at 48 45 -> 26; 1003 -> 1001 at 128 26 -> 21; not
 //    where three launches cost more than that kernel (17..32 tokens 13-22 us, 4097 -> 4096 at
 //    24 14.5 -> 17.1; 511 -> 700 at 65 15.9 -> 17.0);
 //  * where the split of K over tall tiles does not fit the CUs: few tokens (4096 -> 6144 at
-//    65 / 128 / 256 30.4 -> 23.1 / 30.8 -> 25.2 / 35.6 -> 31.6 us, 14336 -> 4096 at 100
-//    56.6 -> 35.0), items past a round (3072 -> 9216 at 600, 270 items, 68.8 -> 51.0) or far
-//    below one (8192 -> 1024 at 512 39.5 -> 30.1).  Where it fits, the split is faster
+//    65 / 128 / 256 30.7 -> 22.1 / 31.3 -> 25.0 / 35.2 -> 31.2 us, 14336 -> 4096 at 100
+//    56.8 -> 30.6), items past a round (3072 -> 9216 at 600, 270 items, 68.8 -> 51.0) or far
+//    below one (8192 -> 1024 at 512 39.8 -> 30.3).  Where it fits, the split is faster
 //    (14336 -> 4096 at 512 68 -> 86, 4096 -> 6144 at 512 43 -> 52), as it is over fewer than
 //    2 Mi weights (1088 -> 1639 at 96 18.7 -> 20.7) and, past 128 tokens, where C takes no
 //    16-byte stores (8768 -> 6781 at 148 46.9 -> 54.7).

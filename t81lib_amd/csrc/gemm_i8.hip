@@ -600,10 +600,10 @@ I8Plan i8_plan(int64_t m, int64_t n, int64_t k) {
 }
 
 // 384 x 128 tiles where they are half a round of the CUs to a whole one, instead of 256 x 256
-// tiles on fewer CUs or their split of K and its int32 sum: 4096 -> 6144 at M = 1536 84.3 ->
-// 48.6 us, at 900 62.3 -> 45.4, at 2048 62.8 -> 56.6; 3072 -> 9216 at 1024 73.9 -> 39.9; 2048 ->
-// 8192 at 777 39.6 -> 32.5.  Over a K past 8192 a split that fits stays faster (14336 -> 4096 at
-// 2048 133 -> 163), so only where there is none (at 2500 tokens 197 -> 167).
+// tiles on fewer CUs or their split of K and its int32 sum: 4096 -> 6144 at M = 1536 85.0 ->
+// 50.8 us, at 900 62.3 -> 44.3, at 2048 61.2 -> 57.9; 3072 -> 9216 at 1024 74.2 -> 38.3; 2048 ->
+// 8192 at 777 40.5 -> 30.9.  Over a K past 8192 a split that fits stays faster (14336 -> 4096 at
+// 2048 133 -> 163), so only where there is none (at 2500 tokens 177 -> 166).
 bool i8_use_384(int64_t m, int64_t n, int64_t k) {
     const int64_t L = (k + kTrits - 1) / kTrits;
     const int64_t t3 = ((n + 383) / 384) * ((m + 127) / 128);

@@ -2,8 +2,9 @@
 //
 //   C[m, n] = alpha * sum_k X[m, k] * T[n, k] + beta * C[m, n] + bias[n]
 //
-// x is cut into P bf16 planes (P = 2: float32 as hi + lo, |x - hi - lo| <= 2^-18 |x|; P = 3:
-// float32 exactly; P = 1: bf16 as it is) by a first small kernel, and the product kernel accumulates every plane's products into the same
+// x is cut into P bf16 planes (P = 2: float32 as hi + lo, |x - hi - lo| <= 2^-17 |x|; P = 3:
+// float32 exactly, but for digits below 2^-133, bf16's smallest value; P = 1: bf16 as it is) by
+// a first small kernel, and the product kernel accumulates every plane's products into the same
 // accumulators: each decoded weight fragment meets P planes before it is dropped, so the
 // trit decode and the weight loads per MFMA are 1 / P of the bf16 kernel's.  What bounds it
 // is the matrix pipe (2 P M N K flops).
@@ -97,8 +98,9 @@ __global__ __launch_bounds__(256) void planes_kernel(
             pl[0][i] = static_cast<__bf16>(v[i]);
             pl[1][i] = static_cast<__bf16>(v[i] - static_cast<float>(pl[0][i]));
         } else if constexpr (P == 3) {
-            // x = hi + mid + lo exactly (8 bits each, round to nearest); |x| past bf16's
-            // largest value rounds to it, not to infinity, and an infinity or NaN is hi alone
+            // x = hi + mid + lo (8 bits each, round to nearest; of |x| < 2^-110 the digits below
+            // 2^-133 are rounded off); |x| past bf16's largest value rounds to it, not to
+            // infinity, and an infinity or NaN is hi alone
             const uint32_t u = __float_as_uint(v[i]);
             const uint32_t mag = u & 0x7FFFFFFFu;
             const bool top = mag >= 0x7F7F8000u;
@@ -693,9 +695,9 @@ hipError_t launch_planes(const void *x, const uint8_t *w, float *c, int64_t m, i
 
 }  // namespace
 
-// Where the planes are taken, against the eight-wave kernel (14336 -> 4096 at M = 1024 833 ->
-// 220 us, 4096 -> 14336 at M = 100 / 512 104 -> 40 / 232 -> 100, at M = 33 / 64 35 -> 26 /
-// 45 -> 33): past 32 tokens, of 33..64 only over 4 Mi weights or a K the vector loads do not
+// Where the planes are taken, against the eight-wave kernel (14336 -> 4096 at M = 1024 828 ->
+// 223 us, 4096 -> 14336 at M = 100 / 512 103 -> 39 / 230 -> 99, at M = 33 / 64 33 -> 26 /
+// 42 -> 32): past 32 tokens, of 33..64 only over 4 Mi weights or a K the vector loads do not
 // take -- three launches cost 14-18 us whatever the size (1000 -> 1000 at 64 tokens 17.6 ->
 // 18.5, at 65 24.6 -> 18.8; 3072 -> 3072 at 64 20.5 -> 18.6), and at 17..32 tokens the
 // eight-wave kernel's 32-token tiles take 13-26 us (4096 -> 14336 at 32 25.4 -> 26.1, 4096 ->
@@ -730,7 +732,7 @@ hipError_t launch_gemm_plane(const void *x, const uint8_t *w, float *c, int64_t 
     return launch_planes<1>(x, w, c, m, n, k, alpha, beta, bias, s, ws);
 }
 
-// Training's product: three planes (x exactly) and a scale in device memory,
+// Training's product: three planes and a scale in device memory,
 //   C[m, n] = *scale * sum_k X[m, k] * T[n, k] + bias[n].
 int64_t gemm_exact_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     return planes_plan(3, m, n, k).bytes;

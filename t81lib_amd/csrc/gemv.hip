@@ -278,7 +278,7 @@ __global__ __launch_bounds__(64 * W) void gemv_wave_kernel(
                 if constexpr (XT == kDtypeBF16) {
                     *reinterpret_cast<u32x4 *>(dst) = raw[i];
                 } else if constexpr (XT == kDtypeF32) {
-                    // x = hi + lo, hi = bf16(x), lo = bf16(x - hi): |x - hi - lo| <= 2^-18 |x|
+                    // x = hi + lo, hi = bf16(x), lo = bf16(x - hi): |x - hi - lo| <= 2^-17 |x|
                     uint32_t h[4], l[4];
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {

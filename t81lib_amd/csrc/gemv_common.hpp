@@ -77,7 +77,7 @@ __device__ __forceinline__ XRaw load_x8_raw(const void *x, int64_t row_off, int6
 }
 
 // bf16 operands of 8 raw activations: bf16 as is; fp32 as x = hi + lo with
-// hi = bf16(x), lo = bf16(x - hi), |x - hi - lo| <= 2^-18 |x|; int8 exactly.
+// hi = bf16(x), lo = bf16(x - hi), |x - hi - lo| <= 2^-17 |x|; int8 exactly.
 template <int XT>
 __device__ __forceinline__ void cvt_x8(const XRaw &raw, bf16x8 &hi, bf16x8 &lo) {
     const u32x4 zero = {0u, 0u, 0u, 0u};

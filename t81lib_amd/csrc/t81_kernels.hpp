@@ -120,7 +120,7 @@ int64_t gemm_plane_workspace_bytes(int64_t m, int64_t n, int64_t k);
 hipError_t launch_gemm_plane(const void *x, const uint8_t *w, float *c, int64_t m, int64_t n,
                              int64_t k, float alpha, float beta, const float *bias,
                              hipStream_t s, void *ws);
-// The same with three planes (x = hi + mid + lo exactly) and a scale in device memory, for
+// The same with three planes (x = hi + mid + lo) and a scale in device memory, for
 // training: C = *scale * X T^T + bias.
 int64_t gemm_exact_workspace_bytes(int64_t m, int64_t n, int64_t k);
 hipError_t launch_gemm_exact(const float *x, const uint8_t *w, float *c, int64_t m, int64_t n,

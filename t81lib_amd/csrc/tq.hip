@@ -97,9 +97,10 @@ __device__ __forceinline__ float wave_max_dpp(float v) {
 // at once.  Their payload bytes are contiguous and go out as dwords through
 // LDS.  kVec: rows are 16-byte aligned runs of whole float4s, else element loads; columns past
 // the row are zeros.  The slots are private to the wavefront (wave_lds_sync, no barrier).
-// 8192 x 3072: TQ1_0 28.2 -> 22.1 us, TQ2_0 25.5 -> 20.7 against one block per wavefront with
-// byte gathers; 8192 x 3008 (partial blocks) 62.7 -> 21.3, 8191 x 3071 64.3 -> 28.7 against
-// strided loads read twice.
+// 8192 x 3072: TQ1_0 29.2 -> 25.0 us, TQ2_0 25.3 -> 21.3 against one block per wavefront with
+// byte gathers; 8192 x 3008 (partial blocks) TQ1_0 63.7 -> 21.8, 8191 x 3071 64.6 -> 28.2
+// against strided loads read twice (calls over eight tensors in turn; from a graph 8192 x 3072
+// takes 21.7 and 21.2).
 template <int Q, bool kVec, int B>
 __global__ __launch_bounds__(256) void tq_quantize_vec_kernel(const float *__restrict__ src,
                                                               uint8_t *__restrict__ dst,
@@ -258,9 +259,9 @@ __global__ __launch_bounds__(256) void tq_quantize_kernel(const float *__restric
 
 // One wavefront per block.  Rows of whole float4s (cols a multiple of 4) into a 16-byte aligned
 // output (kVec): lane l writes weights 4 l .. 4 l + 3 of its block with one non-temporal
-// float4, past the row none (8192 x 3008 TQ1_0 28.4 -> 16.0 us against element stores).
+// float4, past the row none (8192 x 3008 TQ1_0 28.4 -> 18.0 us against element stores).
 // Else the block turns through LDS so that each store is 64 consecutive floats (8191 x 3071
-// TQ1_0 64.3 -> 37.0).  Those four share a digit position: TQ2_0 bits 2s of four
+// TQ1_0 64.5 -> 36.8).  Those four share a digit position: TQ2_0 bits 2s of four
 // consecutive bytes; TQ1_0 digit n of four consecutive bytes (n = e / 32 below 160,
 // (e - 160) / 16 below 240, (e - 240) / 4 after, e = 4 l).
 template <int Q, bool kVec>

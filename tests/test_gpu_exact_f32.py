@@ -23,8 +23,8 @@ by a bit-exact result; float activations enter at t81/torch/__init__.py:241-246)
   K), with the K split over a workspace and without;
 * K3 at M > 64, including the config-4 shape 4096 -> 6144 at M = 512, every output
   against a float64 product of the unpacked trits on the GPU (exact) and a sample
-  against the C oracle; and the path that runs the activations as two bf16 launches of
-  their planes, chunk by chunk, from the workspace.
+  against the C oracle; and the path that runs over an image of their bf16 planes, chunk by
+  chunk, in the workspace.
 """
 
 from __future__ import annotations
@@ -232,11 +232,11 @@ def test_k3_config4_f32_sampled_and_full(gpu, orc):
     torch.cuda.empty_cache()
 
 
-# ------------------------------------------- K3 float32 as two bf16 launches --
+# ------------------------------------------- K3 float32 through its bf16 planes --
 PLANES = [
-    # M, K, N, chunks: float32 activations past 64 tokens whose bf16 launches need no split
-    # of their own run as the bf16 planes in the workspace, chunk by chunk (a chunk's two
-    # planes within 64 MiB): one chunk, and three of 700 tokens over K = 16384
+    # M, K, N, chunks: float32 activations past 32 tokens run through their bf16 planes in the
+    # workspace, by chunks of tokens or parts of K; the reported size holds the two planes of
+    # the fewest equal chunks of tokens within 64 MiB: one, and three of 700 over K = 16384
     (2048, 4096, 6144, 1), (700, 2048, 16384, 1), (2100, 16384, 14336, 3),
 ]
 
@@ -244,9 +244,8 @@ PLANES = [
 @pytest.mark.parametrize("M,K,N,chunks", PLANES)
 def test_k3_f32_planes_bit_exact(gpu, orc, M, K, N, chunks):
     """Every output against a float64 product of the unpacked trits on the GPU (exact), that
-    product against the C oracle on a sample, with the workspace (the planes path: beta and
-    bias in the first launch, the lo plane added by the second) and without it (the
-    eight-wave kernel)."""
+    product against the C oracle on a sample, with the workspace (the planes path: both planes
+    in one launch per chunk) and without it (the eight-wave kernel)."""
     announce(f"exact f32 K3 planes M={M} K={K} N={N}")
     lib = _lib.lib()
     rows = -(-M // chunks)

@@ -5,7 +5,8 @@ Scale, ternarized weight and the weight gradient's passes keep the expression's 
 they are compared bit for bit (NaN as NaN), in each weight type, at the edges of a
 12-weight run, of a limb and of the thresholds.  The products sum in float32 in another
 order: with K terms both sides are within (K + 2) 2^-24 sum |x q s| of the exact value
-(products of the three planes are exact; the expression rounds each product once more),
+(products of the three planes are exact; the expression rounds each product once more; bit
+for bit, in every plane: test_gpu_plane_pairs.py),
 doubled for the matrix cores' own rounding.
 """
 
@@ -205,8 +206,9 @@ PRODUCTS = [(1, 1, 1), (17, 33, 40), (32, 256, 32), (100, 257, 300), (1000, 511,
 @pytest.mark.parametrize("M,N,K", PRODUCTS)
 def test_weight_product(gpu, monkeypatch, M, N, K):
     """Six plane products of M exact terms each, summed in float32: within 2 (6 M + 4) 2^-24
-    sum |g x| (doubled for the matrix cores' rounding); the planes left out are below 2^-26
-    of each term, inside the + 4.  Infinities and NaN as the float32 product gives them."""
+    sum |g x| (doubled for the matrix cores' rounding); the plane products left out are below
+    2^-24 of each term, inside the + 4.  Infinities and NaN as the float32 product gives them.
+    (Bit for bit, in every pair of planes: test_gpu_plane_pairs.py.)"""
     announce(f"qat weight product M={M} N={N} K={K}")
     monkeypatch.setattr(qat, "MIN_WEIGHTS", 0)
     gen = torch.Generator("cpu").manual_seed(M + N + K)
