@@ -356,7 +356,7 @@ int t81_hip_qat_weight_grad(const void *g, int g_dtype, const float *scale,
                             void *stream);
 
 /* c[m, n] = *scale * sum_k x[m, k] * T[n, k] + bias[n], float32, with x split into three bf16
- * planes that hold it exactly, but for digits below 2^-133 (products exact, float32 sums; no
+ * planes that hold it exactly, but for digits below 2^-140 (products exact, float32 sums; no
  * sum overflows where that of x * (*scale * T) does not).  workspace (16-byte aligned):
  * t81_hip_qat_matmul_workspace_size bytes; 0 there: the shape is not taken (EINVAL_SHAPE).
  * Replaces: the F.linear of t81/nn/linear.py:93-99 and its input gradient (with the

@@ -3,11 +3,11 @@
 //   C[m, n] = alpha * sum_k X[m, k] * T[n, k] + beta * C[m, n] + bias[n]
 //
 // x is cut into P bf16 planes (P = 2: float32 as hi + lo, |x - hi - lo| <= 2^-17 |x|; P = 3:
-// float32 exactly, but for digits below 2^-133, bf16's smallest value; P = 1: bf16 as it is) by
-// a first small kernel, and the product kernel accumulates every plane's products into the same
-// accumulators: each decoded weight fragment meets P planes before it is dropped, so the
-// trit decode and the weight loads per MFMA are 1 / P of the bf16 kernel's.  What bounds it
-// is the matrix pipe (2 P M N K flops).
+// float32 exactly, but for digits below 2^-140; P = 1: bf16 as it is) by a first small kernel,
+// and the product kernel accumulates every plane's products into the same accumulators (P = 3:
+// hi's apart from the others'): each decoded weight fragment meets P planes before it is dropped,
+// so the trit decode and the weight loads per MFMA are 1 / P of the bf16 kernel's.  What bounds
+// it is the matrix pipe (2 P M N K flops).
 //
 // Plane image.  The planes are stored piece by piece (8 values of one token, 16 bytes), so a
 // tile load is a straight copy into LDS and a B read is 64 consecutive pieces:
@@ -55,6 +55,11 @@ __device__ __forceinline__ float scale_of_output(const float *scale) {
     return scale == nullptr ? 1.0f : *scale / scale_of_trits(scale);
 }
 
+// Training's mid and lo planes, whose sums are apart from hi's to the end, are stored times 2^7:
+// digits then go down to 2^-140 (bf16's smallest value is 2^-133), and the largest value's mid
+// plane, below 2^120, stays in range.
+constexpr float kSmallPlanes = 128.0f;
+
 // ---- the plane image ----
 // A wave takes 8 tokens x 8 consecutive pieces: it reads 256 contiguous bytes of each token
 // row (K values of ldx) and writes 128 contiguous bytes per piece and plane.
@@ -98,8 +103,8 @@ __global__ __launch_bounds__(256) void planes_kernel(
             pl[0][i] = static_cast<__bf16>(v[i]);
             pl[1][i] = static_cast<__bf16>(v[i] - static_cast<float>(pl[0][i]));
         } else if constexpr (P == 3) {
-            // x = hi + mid + lo (8 bits each, round to nearest; of |x| < 2^-110 the digits below
-            // 2^-133 are rounded off); |x| past bf16's largest value rounds to it, not to
+            // x = hi + mid + lo (8 bits each, round to nearest; of |x| < 2^-117 the digits below
+            // 2^-140 are rounded off); |x| past bf16's largest value rounds to it, not to
             // infinity, and an infinity or NaN is hi alone
             const uint32_t u = __float_as_uint(v[i]);
             const uint32_t mag = u & 0x7FFFFFFFu;
@@ -108,7 +113,9 @@ __global__ __launch_bounds__(256) void planes_kernel(
             if (mag > 0x7F800000u) hb |= 0x40u;
             const uint16_t h16 = static_cast<uint16_t>(hb);
             pl[0][i] = top ? __builtin_bit_cast(__bf16, h16) : static_cast<__bf16>(v[i]);
-            const float r = mag >= 0x7F800000u ? 0.0f : v[i] - static_cast<float>(pl[0][i]);
+            const float r = mag >= 0x7F800000u
+                                ? 0.0f
+                                : (v[i] - static_cast<float>(pl[0][i])) * kSmallPlanes;
             pl[1][i] = static_cast<__bf16>(r);
             pl[2][i] = static_cast<__bf16>(r - static_cast<float>(pl[1][i]));
         }
@@ -399,7 +406,8 @@ __global__ __launch_bounds__(256) void gemm_planes_kernel(
 #pragma unroll
                 for (int j = 0; j < CB; ++j)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) acc[i][j][v] += acc[i][j + CB][v];
+                    for (int v = 0; v < 16; ++v)
+                        acc[i][j][v] += acc[i][j + CB][v] * (1.0f / kSmallPlanes);
         }
 
         // ---- epilogue: through the wave's LDS region, 32 tokens x 64 rows at a time, so a

@@ -15,7 +15,7 @@ seeded run repeats.  Plain torch code, on whatever device the tensors are on.
 ternary(w / s) * s, b)``, for ``t8.nn.Linear``'s training step on the GPU (csrc/qat.hip): the
 weight and its gradient take one pass each instead of about twenty-five, and a float32
 product runs over the packed trits with the activations split into three bf16 planes
-(exactly, but for digits below 2^-133).  Results keep the tensor expression's roundings (weights and
+(exactly, but for digits below 2^-140).  Results keep the tensor expression's roundings (weights and
 weight-gradient passes bit for bit); ``weight_on_kernels`` and ``product_on_kernels`` say when
 they stand in, everything else (other devices, subclasses, tracing, modes, forward-mode) runs
 the expression itself.

@@ -10,7 +10,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from t81lib_amd import qat
+from t81lib_amd import ops, qat
 from test_gpu_exact_f32 import announce
 from test_gpu_qat import PRODUCTS, U32, expression, expression_scale, layers
 
@@ -69,6 +69,28 @@ def test_weight_product_small_values(gpu, monkeypatch, M, N, K):
     for g, v in ((one.to(gpu), x), (x, one.to(gpu))):
         got, want = qat.weight_product(g, v), g.double().T @ v.double()
         assert torch.equal(got.double(), want)
+
+
+@pytest.mark.parametrize("M,K,N", [(70, 97, 513), (100, 1001, 300), (96, 6000, 130)])
+def test_training_product_small_and_large_values(gpu, M, K, N):
+    """One term per output: values whose digits end at 2^-140 or above, up to the largest, are
+    held to the last bit."""
+    announce(f"qat product small values M={M} K={K} N={N}")
+    gen = torch.Generator("cpu").manual_seed(M + N * 3 + K)
+    exps = torch.where(torch.rand((M, K), generator=gen) < 0.5,
+                       torch.randint(-140, -100, (M, K), generator=gen),
+                       torch.randint(60, 105, (M, K), generator=gen)).double()
+    x = (torch.randint(1, 1 << 24, (M, K), generator=gen).double() * 2.0 ** exps).float()
+    x[:, 0], x[:, 1] = 3.4028234e38, -3.3953138e38  # the largest float32, and past bf16's
+    t = torch.zeros((N, K))
+    at = torch.randint(0, K, (N,), generator=gen)
+    at[0], at[1] = 0, 1
+    t[torch.arange(N), at] = 1.0
+    x, packed = x.to(gpu), ops.quantize_pack(t.to(gpu), 0.5)
+    for s in (1.0, 0.5):
+        got = qat._matmul(x, packed, N, torch.tensor(s, device=gpu), None)
+        want = (s * x.double()[:, at.to(gpu)])
+        assert torch.equal(got.double(), want.float().double())
 
 
 @pytest.mark.parametrize("std", [0.02, 30.0])
