@@ -128,3 +128,35 @@ def test_training_product_overflow(gpu, monkeypatch, M, K, N, std):
         assert not bool(got.isnan().any())
         bound = 2.0 * (a.shape[1] + 2) * U32 * mags + 1e-30
         assert bool(((got - want).abs() <= bound)[sure].all())
+
+
+def test_weight_product_under_graph_capture(gpu, monkeypatch):
+    """The note of large values is the launch's own: replays on inputs that turn large and back
+    equal the eager results, with eager work between them."""
+    announce("qat weight product graph capture")
+    monkeypatch.setattr(qat, "MIN_WEIGHTS", 0)
+    M, N, K = 1040, 130, 64  # (the tokens split)
+    torch.manual_seed(9)
+    g, x = torch.randn((M, N), device=gpu), torch.randn((M, K), device=gpu)
+    plain = x.clone()
+    large = x.clone()
+    large[5, 7] = 1e20
+    infinite = x.clone()
+    infinite[5, 7] = float("inf")
+    want = {}
+    for name, v in (("plain", plain), ("large", large), ("infinite", infinite)):
+        want[name] = qat.weight_product(g, v)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = qat.weight_product(g, x)
+    for name, v in (("large", large), ("plain", plain), ("infinite", infinite), ("plain", plain),
+                    ("plain", plain), ("large", large)):
+        x.copy_(v)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        same = (out == want[name]) | (out.isnan() & want[name].isnan())
+        assert bool(same.all()), name
+        other = qat.weight_product(g, infinite)  # eager work in between
+        del other
+    del graph
