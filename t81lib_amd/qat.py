@@ -90,11 +90,9 @@ def observed() -> bool:
             torch.autograd.forward_ad._current_level >= 0)
 
 
-def _plain(*tensors: Optional[torch.Tensor]) -> bool:
-    """Ordinary contiguous tensors on the current GPU, and nothing that observes.  (A batch of
-    gradients taken through one graph at once has no storage of its own.)"""
-    if observed():
-        return False
+def _ordinary(*tensors: Optional[torch.Tensor]) -> bool:
+    """Contiguous tensors on the current GPU, of no subclass.  (A batch of gradients taken through
+    one graph at once has no storage of its own.)"""
     for t in tensors:
         if t is None:
             continue
@@ -107,9 +105,14 @@ def _plain(*tensors: Optional[torch.Tensor]) -> bool:
     return True
 
 
+def _plain(*tensors: Optional[torch.Tensor]) -> bool:
+    """Ordinary tensors, and nothing that observes."""
+    return not observed() and _ordinary(*tensors)
+
+
 def _as_saved(t: torch.Tensor, dtype: torch.dtype, *shape: int) -> bool:
     """Whether a saved tensor came back as it was (saved-tensor hooks may return another)."""
-    return t.dtype == dtype and t.shape == shape and _plain(t)
+    return t.dtype == dtype and t.shape == shape and _ordinary(t)
 
 
 def weight_on_kernels(weight: torch.Tensor, threshold: float) -> bool:
@@ -137,7 +140,8 @@ def product_on_kernels(x: torch.Tensor, weight: torch.Tensor,
 
 
 def scale_on_kernels(existing: Optional[torch.Tensor]) -> bool:
-    return existing is None or (_plain(existing) and existing.ndim == 0 and
+    """(asked where weight_on_kernels holds)"""
+    return existing is None or (_ordinary(existing) and existing.ndim == 0 and
                                 existing.dtype == torch.float32 and not existing.requires_grad)
 
 
